@@ -301,6 +301,26 @@ void build_lut(Codebook& book) {
     }
     for (size_t i = 0; i < esc.size(); ++i)
         tokens[i] = (book.token_bytes[esc[i]] & 0xFFFFu) | (Codebook::token_width(esc[i]) << NZ_ENTRY_COUNT);
+    // escape prefixes (see nz_format.h)
+    const uint32_t first_token = NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * lut[0];
+    for (uint32_t x = 0; x < NZ_LUT_ENTRIES; ++x) {
+        if (single[x] >= 0) continue;
+        // first and last codes under the prefix (canonical codes increase with their length)
+        unsigned lo = 0, hi = 0;
+        while (lo + 1 < esc.size() && book.codes[esc[lo]] >> (book.lengths[esc[lo]] - NZ_LUT_BITS) < x) ++lo;
+        hi = lo;
+        while (hi + 1 < esc.size() && book.codes[esc[hi + 1]] >> (book.lengths[esc[hi + 1]] - NZ_LUT_BITS) == x) ++hi;
+        const unsigned L = book.lengths[esc[lo]];
+        uint32_t* entry = &lut[NZ_LUT_HEADER + 2 * x];
+        if (L == book.lengths[esc[hi]] && L <= 32) {
+            entry[0] = 32u - L;
+            entry[1] = first_token + lo;
+        } else {
+            const auto at = std::find(esc_lengths.begin(), esc_lengths.end(), L);
+            entry[0] = NZ_ESC_SEARCH;
+            entry[1] = static_cast<uint32_t>(at - esc_lengths.begin());
+        }
+    }
     check_lut_image(lut);
 }
 
@@ -344,6 +364,11 @@ unsigned lut_step(const std::vector<uint32_t>& lut, uint64_t window, uint32_t* b
     const uint64_t end = k + 1 < n_len ? word(k + 1, 4) : n_tokens;   // tokens of length L end here
     if (word(k, 4) + offset >= end)
         fail(kCorruptStream, "Escape token index past its code length's tokens.");
+    // the primary entry's shortcut must lead to the same length and token
+    if (e < NZ_ESC_SEARCH
+            ? L != 32u - e || e1 + ((window << NZ_LUT_BITS) >> (NZ_LUT_BITS + 64 - L)) != tokens + word(k, 4) + offset
+            : e1 > k || (e1 && window < (word(e1 - 1, 0) | static_cast<uint64_t>(word(e1 - 1, 1)) << 32)))
+        fail(kCorruptStream, "Escape entry does not lead to its code's token.");
     const uint32_t te = lut.at(tokens + word(k, 4) + offset);
     *bytes = te & 0xFFFFu;
     *count = te >> NZ_ENTRY_COUNT;

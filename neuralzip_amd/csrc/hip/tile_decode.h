@@ -66,13 +66,13 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// Canonical decode of one code longer than 12 bits: find the first escape
-// length whose left-justified limit exceeds the window. Returns the escape
-// token entry; *len receives the code length.
-__device__ __forceinline__ uint32_t escape_entry(const uint32_t* lut, uint64_t window, uint32_t* len) {
+// Canonical decode of one code longer than 12 bits whose prefix holds codes
+// of several lengths: from record `k` on, find the first escape length whose
+// left-justified limit exceeds the window. Returns the escape token entry;
+// *len receives the code length.
+__device__ __forceinline__ uint32_t escape_search(const uint32_t* lut, uint64_t window, uint32_t k, uint32_t* len) {
     const uint32_t n_len = lut[0];
     const uint32_t* rec = lut + NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES;
-    uint32_t k = 0;
     while (k + 1 < n_len) {
         const uint64_t limit = rec[NZ_ESC_RECORD * k] | (static_cast<uint64_t>(rec[NZ_ESC_RECORD * k + 1]) << 32);
         if (window < limit) break;
@@ -254,29 +254,45 @@ __device__ __forceinline__ void fetch(const TileInfo& ti, uint32_t lane, Fetch<E
     fetch_raw<ES, LONG>(ti, lane, d);
 }
 
-// One LUT step at the head of the window w0..w3: returns the entry (byte
-// count in bits 27-29 of .x; the bytes, first lowest and zeros above them,
-// in .y) and shifts the window by the consumed bits.
+__device__ __forceinline__ uint2 lut_entry(const uint32_t* lut, uint32_t w0) {
+    return reinterpret_cast<const uint2*>(lut + NZ_LUT_HEADER)[w0 >> (32 - NZ_LUT_BITS)];
+}
+
+// One LUT step at the head of the window w0..w3, whose primary entry is `e`:
+// returns the step's entry (byte count in bits 27-29 of .x; the bytes, first
+// lowest and zeros above them, in .y) and shifts the window by the consumed
+// bits.
 template <bool LONG, bool ESC>
-__device__ __forceinline__ uint2 lut_step(const uint32_t* lut, uint32_t& w0, uint32_t& w1, uint32_t& w2,
+__device__ __forceinline__ uint2 lut_step(const uint32_t* lut, uint2 e, uint32_t& w0, uint32_t& w1, uint32_t& w2,
                                           uint32_t& w3) {
-    uint2 e = reinterpret_cast<const uint2*>(lut + NZ_LUT_HEADER)[w0 >> (32 - NZ_LUT_BITS)];
     uint32_t s = e.x;   // the funnel shift reads its low five bits
     if (ESC) {
-        // wave-uniform test first (one compare into a lane mask): escapes are rare
-        if (__builtin_amdgcn_uicmp(e.x, 1u << NZ_ENTRY_COUNT, kIcmpUlt)) {
+        // One scalar branch where no lane escapes (0.5 % of a lane's steps
+        // do, so three steps in ten of a wavefront); the empty asm keeps the
+        // compiler from folding the lanes' test into it. An escape entry
+        // names the token of almost every escape, one LDS read: searching
+        // the length records for each one took 35 % of the fused kernel's
+        // vector instructions and 65 % of its scalar ones (58.7 M bf16
+        // elements, 59.2 -> 51.0 us for the product).
+        if (__builtin_expect(__builtin_amdgcn_uicmp(e.x, 1u << NZ_ENTRY_COUNT, kIcmpUlt) != 0, 0)) {
+            asm volatile("");
             if (e.x < (1u << NZ_ENTRY_COUNT)) {
-                uint32_t len;
-                e.x = escape_entry(lut, (static_cast<uint64_t>(w0) << 32) | w1, &len);
-                e.y = e.x & 0xFFFFu;   // one or two bytes
-                if (LONG && len > 32) {
-                    w0 = w1;
-                    w1 = w2;
-                    w2 = w3;
-                    w3 = 0;
-                    len -= 32;
+                if (e.x < NZ_ESC_SEARCH) {
+                    // the code's bits past the prefix count up from the prefix's first token
+                    e.x = lut[e.y + ((w0 << NZ_LUT_BITS) >> (NZ_LUT_BITS + s))];
+                } else {
+                    uint32_t len;
+                    e.x = escape_search(lut, (static_cast<uint64_t>(w0) << 32) | w1, e.y, &len);
+                    if (LONG && len > 32) {
+                        w0 = w1;
+                        w1 = w2;
+                        w2 = w3;
+                        w3 = 0;
+                        len -= 32;
+                    }
+                    s = 32 - len;   // len in [1, 32]; s == 0 shifts a whole word
                 }
-                s = 32 - len;   // len in [1, 32]; s == 0 shifts a whole word
+                e.y = e.x & 0xFFFFu;   // one or two bytes
             }
         }
     }
@@ -334,8 +350,12 @@ __device__ __forceinline__ void stage_tile(const TileInfo& ti, const Fetch<ES, L
             reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)stage));
         uint32_t bit = 8 * (base + at);
         const uint32_t stop = bit + 8 * count;
+        // The next step's LUT read is issued before this step's ORs, so that
+        // its latency covers theirs; the last one's entry goes unused.
+        uint2 e = lut_entry(lut, w0);
         do {
-            const uint2 e = lut_step<LONG, ESC>(lut, w0, w1, w2, w3);
+            e = lut_step<LONG, ESC>(lut, e, w0, w1, w2, w3);
+            const uint2 next = lut_entry(lut, w0);
             lds_u32* dst = (lds_u32*)(uintptr_t)((bit >> 3) & ~3u);
             // The entry's bytes in this dword, and the ones past it: one
             // 64-bit shift (two 32-bit shifts and a negation before).
@@ -344,13 +364,13 @@ __device__ __forceinline__ void stage_tile(const TileInfo& ti, const Fetch<ES, L
             const uint32_t high = static_cast<uint32_t>(both >> 32);
             __hip_atomic_fetch_or(dst, low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             __hip_atomic_fetch_or(dst + 1, high, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            // The ORs complete before the wavefront issues its next LDS
-            // instruction (the next LUT read). On gfx950 an LDS read issued
-            // while the same wavefront's LDS atomics were still in flight has
-            // returned staging data in place of the LUT entry, now and then;
-            // waiting here costs under 1 % of the decode time.
+            // The read and the ORs complete before the wavefront issues its
+            // next LDS instruction. On gfx950 an LDS read issued while the
+            // same wavefront's LDS atomics were still in flight has returned
+            // staging data in place of the LUT entry, now and then.
             __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
             bit += e.x >> (NZ_ENTRY_COUNT - 3);   // 8 x the byte count (bits 5-26 of an entry are zero)
+            e = next;
         } while (bit < stop);
     }
     wave_lds_sync();

@@ -60,11 +60,17 @@
 // bits), and its top byte is 8 x the byte count, which one byte-select add
 // (SDWA) adds to a bit position; word 1 is stored as one dword.
 // Escape token entry: b0 | b1 << 8 | byte count << 27.
+// An escape's primary entry (byte count 0) saves the kernels the search of
+// the records: where all codes under the prefix have one length L <= 32,
+//   word 0: 32 - L      word 1: image word of the token of its first code
+// (the code's L - 12 bits past the prefix count up from there), else
+//   word 0: NZ_ESC_SEARCH      word 1: the record the search starts at.
 #define NZ_LUT_HEADER 4
 #define NZ_ESC_RECORD 6
 #define NZ_ENTRY_SHIFT_MASK 31u
 #define NZ_ENTRY_COUNT 27
 #define NZ_ENTRY_MAX_BYTES 4
+#define NZ_ESC_SEARCH 64u
 #define NZ_LUT_MAX_WORDS (NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * 56 + 512)
 
 enum nz_kind : uint32_t { NZ_KIND_RAW = 0, NZ_KIND_SHORT = 1, NZ_KIND_LONG = 2 };
