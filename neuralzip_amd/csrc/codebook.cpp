@@ -310,10 +310,12 @@ void build_lut(Codebook& book) {
         while (lo + 1 < esc.size() && book.codes[esc[lo]] >> (book.lengths[esc[lo]] - NZ_LUT_BITS) < x) ++lo;
         hi = lo;
         while (hi + 1 < esc.size() && book.codes[esc[hi + 1]] >> (book.lengths[esc[hi + 1]] - NZ_LUT_BITS) == x) ++hi;
-        const unsigned L = book.lengths[esc[lo]];
+        const unsigned L = book.lengths[esc[lo]], last = book.lengths[esc[hi]];
+        unsigned n = 0;   // codes of the first length; the others must all have the last one's
+        while (lo + n <= hi && book.lengths[esc[lo + n]] == L) ++n;
         uint32_t* entry = &lut[NZ_LUT_HEADER + 2 * x];
-        if (L == book.lengths[esc[hi]] && L <= 32) {
-            entry[0] = 32u - L;
+        if (last <= 32 && (L == last || book.lengths[esc[lo + n]] == last)) {
+            entry[0] = (44u - L) | (44u - last) << NZ_ESC_SECOND | (L == last ? NZ_ESC_ALL : n) << NZ_ESC_COUNT;
             entry[1] = first_token + lo;
         } else {
             const auto at = std::find(esc_lengths.begin(), esc_lengths.end(), L);
@@ -365,10 +367,20 @@ unsigned lut_step(const std::vector<uint32_t>& lut, uint64_t window, uint32_t* b
     if (word(k, 4) + offset >= end)
         fail(kCorruptStream, "Escape token index past its code length's tokens.");
     // the primary entry's shortcut must lead to the same length and token
-    if (e < NZ_ESC_SEARCH
-            ? L != 32u - e || e1 + ((window << NZ_LUT_BITS) >> (NZ_LUT_BITS + 64 - L)) != tokens + word(k, 4) + offset
-            : e1 > k || (e1 && window < (word(e1 - 1, 0) | static_cast<uint64_t>(word(e1 - 1, 1)) << 32)))
+    if (e != NZ_ESC_SEARCH) {
+        const uint32_t rest = static_cast<uint32_t>(window >> 32) << NZ_LUT_BITS;
+        const uint32_t n = (e >> NZ_ESC_COUNT) & NZ_ESC_ALL;
+        uint32_t shift = e & 31u, at = rest >> shift;
+        if (at >= n) {
+            const uint32_t second = (e >> NZ_ESC_SECOND) & 31u;
+            at = n + (rest >> second) - (n << (shift - second));
+            shift = second;
+        }
+        if (L != 44u - shift || e1 + at != tokens + word(k, 4) + offset)
+            fail(kCorruptStream, "Escape entry does not lead to its code's token.");
+    } else if (e1 > k || (e1 && window < (word(e1 - 1, 0) | static_cast<uint64_t>(word(e1 - 1, 1)) << 32))) {
         fail(kCorruptStream, "Escape entry does not lead to its code's token.");
+    }
     const uint32_t te = lut.at(tokens + word(k, 4) + offset);
     *bytes = te & 0xFFFFu;
     *count = te >> NZ_ENTRY_COUNT;

@@ -42,11 +42,10 @@ constexpr int kHalfWaves = 8;
 // two workgroups per CU allows 8 at 16 wavefronts per group and 4 at 8.
 constexpr int waves_per_eu(int waves) { return waves == kWaves ? 8 : 4; }
 
-// One element from its exponent byte and its raw lane bytes `raw`
-// (lane k in byte k).
+// One element from its staged exponent byte and its raw lane bytes.
 template <int ES, bool REORDER>
-__device__ __forceinline__ void store_element(uint8_t* out, uint32_t expo, uint32_t raw) {
-    const uint32_t v = restore_word<ES, REORDER>((expo << (8 * (ES - 1))) | raw);
+__device__ __forceinline__ void store_element(uint8_t* out, uint32_t staged, uint32_t raw) {
+    const uint32_t v = element_word<ES, REORDER>(staged, raw);
     if (ES == 2) {
         *reinterpret_cast<uint16_t*>(out) = static_cast<uint16_t>(v);
     } else {
@@ -56,8 +55,8 @@ __device__ __forceinline__ void store_element(uint8_t* out, uint32_t expo, uint3
 
 // The same through a buffer resource (offset kOutOfRange stores nothing).
 template <int ES, bool REORDER>
-__device__ __forceinline__ void store_element(rsrc_t out, uint32_t offset, uint32_t expo, uint32_t raw) {
-    const uint32_t v = restore_word<ES, REORDER>((expo << (8 * (ES - 1))) | raw);
+__device__ __forceinline__ void store_element(rsrc_t out, uint32_t offset, uint32_t staged, uint32_t raw) {
+    const uint32_t v = element_word<ES, REORDER>(staged, raw);
     if (ES == 2) {
         __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(v), out, offset, 0, 0);
     } else {
@@ -66,15 +65,15 @@ __device__ __forceinline__ void store_element(rsrc_t out, uint32_t offset, uint3
 }
 
 
-// Decodes a tile and stores its words into the workspace `out`: streaming
-// (nontemporal) stores, or, with CACHED, ordinary stores that leave the words
-// in the caches for a consumer that runs right after the decode.
-template <int ES, bool REORDER, bool LONG, bool ESC, bool CACHED>
-__device__ __forceinline__ void huffman_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, const uint32_t* lut,
-                                             uint8_t* stage, uint32_t lane, uint8_t* out_base) {
+// Merges a decoded tile's staged exponents with its raw lanes and stores the
+// words into the workspace `out`: streaming (nontemporal) stores, or, with
+// CACHED, ordinary stores that leave the words in the caches for a consumer
+// that runs right after the decode.
+template <int ES, bool REORDER, bool LONG, bool CACHED>
+__device__ __forceinline__ void store_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, const uint8_t* stage,
+                                           uint32_t lane, uint8_t* out_base) {
     using G = Geometry<ES>;
     constexpr uint32_t V = G::V;
-    stage_tile<ES, LONG, ESC>(ti, d, lut, stage, lane);
     // Every lane issues every store; lanes without a whole vector (or edge
     // element) aim outside the buffer range and store nothing, so the
     // number of memory instructions per tile is fixed and waiting for the
@@ -83,8 +82,9 @@ __device__ __forceinline__ void huffman_tile(const TileInfo& ti, const Fetch<ES,
 #pragma unroll
     for (uint32_t r = 0; r < G::kRounds; ++r) {
         const uint32_t g = (lane + NZ_WAVE * r) * V;
-        const bool whole = g >= ti.s0 && g + V <= ti.s1;
-        const uint8_t* at = stage + NZ_STAGE_ORIGIN + (whole ? g : 0u);
+        // (the round's first element on the scalar side of the comparison)
+        const bool whole = g >= ti.s0 && static_cast<int32_t>(lane * V) <= static_cast<int32_t>(ti.s1 - V - r * NZ_WAVE * V);
+        const uint8_t* at = stage + NZ_STAGE_ORIGIN + g;
         uint32_t e0, e1 = 0;
         if (ES == 2) {
             const uint2 e = *reinterpret_cast<const uint2*>(at);
@@ -135,13 +135,14 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_frag_desc& f
                 r[1] = *reinterpret_cast<const uint32_t*>(lanes + f.lane_stride);
                 r[2] = *reinterpret_cast<const uint32_t*>(lanes + 2 * f.lane_stride);
             }
-            *reinterpret_cast<uint4*>(out + g * ES) = merge_vector<ES, REORDER>(e0, e1, r);
+            *reinterpret_cast<uint4*>(out + g * ES) =
+                merge_vector<ES, REORDER>(staged_form<REORDER>(e0), staged_form<REORDER>(e1), r);
         } else {
             for (uint32_t j = 0; j < V; ++j) {
                 if (g + j >= A0 && g + j < A1) {
                     uint32_t raw = 0;
                     for (int k = 0; k + 1 < ES; ++k) raw |= static_cast<uint32_t>(lanes[j + k * f.lane_stride]) << (8 * k);
-                    store_element<ES, REORDER>(out + (g + j) * ES, expo[j], raw);
+                    store_element<ES, REORDER>(out + (g + j) * ES, staged_form<REORDER>(expo[j]) & 0xFFu, raw);
                 }
             }
         }
@@ -156,19 +157,29 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_fr
                                                 const nz_work& seg, uint32_t* counter, uint32_t lane,
                                                 const uint32_t* lut, uint8_t* stage, uint8_t* out) {
     const uint32_t n = seg.tile1 - seg.tile0;
-    uint32_t t = claim(counter, lane);
+    uint32_t t = claim(counter);
     if (t >= n) return;
     TileInfo cur = tile_info<ES>(base, frags, tiles, seg.tile0 + t);
     Fetch<ES, LONG> fc;
-    fetch<ES, LONG>(cur, lane, fc);
-    uint32_t tn = claim(counter, lane);
+    fetch_bits<ES, LONG>(cur, lane, fc);
+    // Raw lanes are requested a tile ahead, but for long codes of 32-bit
+    // words, where the next tile's twelve registers would spill.
+    constexpr bool kAhead = !(ES == 4 && LONG);
+    if (kAhead) fetch_raw<ES, LONG>(cur, lane, fc);
+    uint32_t tn = claim(counter);
     for (;;) {
         const bool more = tn < n;
         const TileInfo nxt = tile_info<ES>(base, frags, tiles, seg.tile0 + (more ? tn : t));
         Fetch<ES, LONG> fn;
-        fetch<ES, LONG>(nxt, lane, fn);
-        const uint32_t after = more ? claim(counter, lane) : n;
-        huffman_tile<ES, REORDER, LONG, ESC, CACHED>(cur, fc, lut, stage, lane, out);
+        if (kAhead)
+            fetch_raw<ES, LONG>(nxt, lane, fn);
+        else
+            fetch_raw<ES, LONG>(cur, lane, fc);
+        const uint32_t after = more ? claim(counter) : n;
+        const LaneDecode l = open_tile<ES, LONG>(cur, fc, stage, lane);
+        fetch_bits<ES, LONG>(nxt, lane, fn);   // into the registers the open tile no longer needs
+        decode_tile<LONG, ESC>(l, lut);
+        store_tile<ES, REORDER, LONG, CACHED>(cur, fc, stage, lane, out);
         if (!more) break;
         t = tn;
         tn = after;
@@ -181,7 +192,7 @@ template <int ES, bool REORDER>
 __device__ __forceinline__ void raw_segment(const uint8_t* base, const nz_frag_desc* frags, const nz_tile* tiles,
                                             const nz_work& seg, uint32_t* counter, uint32_t lane, uint8_t* out) {
     const uint32_t n = seg.tile1 - seg.tile0;
-    for (uint32_t t = claim(counter, lane); t < n; t = claim(counter, lane)) {
+    for (uint32_t t = claim(counter); t < n; t = claim(counter)) {
         const nz_tile tile = tiles[seg.tile0 + t];
         const nz_frag_desc f = frags[tile.frag];
         raw_tile<ES, REORDER>(base, f, tile, lane, out);
@@ -196,38 +207,30 @@ __global__ __launch_bounds__(WAVES * NZ_WAVE) __attribute__((amdgpu_waves_per_eu
 void nz_decode_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __restrict__ frags,
                       const nz_tile* __restrict__ tiles, const nz_work* __restrict__ segs,
                       uint8_t* __restrict__ out) {
-    using G = Geometry<ES>;
-    __shared__ __align__(16) uint32_t s_lut[NZ_LUT_MAX_WORDS];
-    __shared__ __align__(16) uint8_t s_stage[WAVES][G::kStage];
-    __shared__ uint32_t s_claim;
+    __shared__ __align__(16) GroupLds<ES, WAVES> lds;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NZ_WAVE);
-    const uint32_t lane = threadIdx.x % NZ_WAVE;
+    const uint32_t lane = lane_index();
     const nz_work seg = segs[blockIdx.x];
-    if (threadIdx.x == 0) s_claim = 0;
+    if (threadIdx.x == 0) lds.claim[0] = 0;
     if (seg.kind == NZ_KIND_RAW) {
         __syncthreads();
-        raw_segment<ES, REORDER>(base, frags, tiles, seg, &s_claim, lane, out);
+        raw_segment<ES, REORDER>(base, frags, tiles, seg, lds.claim, lane, out);
         return;
     }
-    const uint4* img = reinterpret_cast<const uint4*>(base + frags[seg.lut_frag].lut);
-    // the host checks every image against NZ_LUT_MAX_WORDS; the clamp keeps a
-    // malformed one from overwriting the staging areas behind s_lut
-    const uint32_t words = min(reinterpret_cast<const uint32_t*>(img)[2], uint32_t(NZ_LUT_MAX_WORDS));
-    uint4* dst = reinterpret_cast<uint4*>(s_lut);
-    for (uint32_t i = threadIdx.x; i < (words + 3) / 4; i += WAVES * NZ_WAVE) dst[i] = img[i];
+    load_lut<REORDER, WAVES * NZ_WAVE>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
     __syncthreads();
     // Codebooks whose codes all fit the primary table run the loop without
     // the escape check (long-code codebooks always have escapes).
     if constexpr (LONG) {
-        huffman_segment<ES, REORDER, true, true, CACHED>(base, frags, tiles, seg, &s_claim, lane, s_lut, s_stage[wave],
+        huffman_segment<ES, REORDER, true, true, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut, lds.stage[wave],
                                                          out);
     } else {
-        if (s_lut[0])
-            huffman_segment<ES, REORDER, false, true, CACHED>(base, frags, tiles, seg, &s_claim, lane, s_lut,
-                                                              s_stage[wave], out);
+        if (lds.lut[0])
+            huffman_segment<ES, REORDER, false, true, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut,
+                                                              lds.stage[wave], out);
         else
-            huffman_segment<ES, REORDER, false, false, CACHED>(base, frags, tiles, seg, &s_claim, lane, s_lut,
-                                                               s_stage[wave], out);
+            huffman_segment<ES, REORDER, false, false, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut,
+                                                               lds.stage[wave], out);
     }
 }
 

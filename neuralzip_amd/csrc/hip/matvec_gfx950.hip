@@ -36,11 +36,11 @@
 namespace {
 
 // Wavefronts per workgroup of the fused kernel, by activation rows: 16 (eight
-// per SIMD within 64 VGPRs) for one row; 12 (six per SIMD within 80 VGPRs)
-// for two to four, whose accumulators and activation vectors spill at 64.
-// Either way two workgroups share a CU's LDS.
+// per SIMD within 64 VGPRs) for one or two rows; 12 (six per SIMD within 80
+// VGPRs) for three or four, whose accumulators and activation vectors spill
+// at 64. Either way two workgroups share a CU's LDS.
 template <int BT>
-constexpr int matvec_waves() { return BT == 1 ? 16 : 12; }
+constexpr int matvec_waves() { return BT <= 2 ? 16 : 12; }
 template <int BT>
 constexpr int matvec_threads() { return matvec_waves<BT>() * NZ_WAVE; }
 constexpr int kReduceThreads = 256;
@@ -95,8 +95,10 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xF, 0xF, false));
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, false));
     v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
+    // rows 1 and 3 add row 0's and row 2's last lane, then rows 2 and 3 add
+    // lane 31 (the wait states that DPP reads of a fresh result need included)
+    asm("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf" : "+v"(v));
     return v;
 }
 
@@ -150,7 +152,7 @@ struct Partial {
     // positions `entry` and, when the tile reaches the next row (`two`),
     // entry + 1 (every other lane's stores fall outside the buffer range).
     // Without `two`, position entry + 1 belongs to the next tile.
-    __device__ __forceinline__ void flush(rsrc_t partials, const RowSpan& rs, bool two, uint32_t batch,
+    __device__ __forceinline__ void flush(float* __restrict__ partials, const RowSpan& rs, bool two, uint32_t batch,
                                           uint32_t lane) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
@@ -158,56 +160,112 @@ struct Partial {
             for (int b = 0; b < BT; ++b) {
                 if (s == 1 && !two) break;
                 const float total = wave_sum(acc[s][b]);
-                const uint32_t at = ((rs.entry + s) * batch + b) * 4u;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(total), partials,
-                                                      lane == NZ_WAVE - 1 && b < static_cast<int>(batch) ? at : kOutOfRange,
-                                                      0, 0);
+                if (lane == NZ_WAVE - 1 && b < static_cast<int>(batch)) partials[(rs.entry + s) * batch + b] = total;
             }
     }
 };
 
-// Adds the products of a tile's staged elements (Huffman tiles) to `p`.
+// One activation row per batch row: a buffer resource over its cols elements.
+template <int BT>
+struct Activations {
+    rsrc_t row[BT];
+};
+
+template <int ES, int BT>
+__device__ __forceinline__ Activations<BT> activations(const uint8_t* xp, uint32_t cols, uint32_t batch) {
+    Activations<BT> a;
+#pragma unroll
+    for (uint32_t b = 0; b < BT; ++b)   // rows past the batch repeat row 0; their sums are never stored
+        a.row[b] = make_rsrc(xp + static_cast<uint64_t>(b < batch ? b : 0u) * cols * ES, cols * ES);
+    return a;
+}
+
+// The activations of rounds R0 to R1 - 1 of one tile, for this lane. Round r's
+// vector starts at column col0 + g of the tile's first row or, past its end,
+// of the next one: the smaller of the offset and the offset less a row, which
+// wraps round to a huge number in the first row. A tile of one row (most
+// tiles) needs one address for all rounds. Lanes past the tile read columns
+// that go unused.
+template <int ES, int BT, uint32_t R0, uint32_t R1>
+__device__ __forceinline__ void fetch_x(const Activations<BT>& x, const RowSpan& rs, const TileInfo& ti, uint32_t cols,
+                                        uint32_t lane, uint4 (*out)[BT]) {
+    const uint32_t at = rs.col0 * ES + lane * 16u;
+    if (rs.split < ti.s1) {
+        asm volatile("");
+#pragma unroll
+        for (uint32_t r = R0; r < R1; ++r) {
+            const uint32_t a = at + r * NZ_WAVE * 16u;
+#pragma unroll
+            for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], min(a, a - cols * ES));
+        }
+    } else {
+        asm volatile("");
+#pragma unroll
+        for (uint32_t r = R0; r < R1; ++r)
+#pragma unroll
+            for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], at + r * NZ_WAVE * 16u);
+    }
+}
+
+template <int ES, int BT>
+__device__ __forceinline__ void fetch_x_round(const Activations<BT>& x, const RowSpan& rs, const TileInfo& ti,
+                                              uint32_t cols, uint32_t lane, uint32_t r, uint4 (&out)[BT]) {
+    const uint32_t a = rs.col0 * ES + lane * 16u + r * NZ_WAVE * 16u;
+    const uint32_t at = rs.split < ti.s1 ? min(a, a - cols * ES) : a;
+#pragma unroll
+    for (int b = 0; b < BT; ++b) out[b] = load_vector(x.row[b], at);
+}
+
+// Rounds whose activations are requested before the tile's decode.
+template <int BT>
+constexpr uint32_t early_rounds() { return BT == 1 ? 2 : 1; }
+
+// Adds the products of a tile's staged elements (Huffman tiles) to `p`: one
+// round per 64 vectors. What holds for a whole round (all vectors inside the
+// tile, all on one side of the row split, none at all) is decided by scalar
+// branches; only a round that the tile's end or the split cuts masks lanes.
 template <int ES, bool REORDER, bool LONG, int BT>
 __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, const uint8_t* stage,
-                                              const RowSpan& rs, rsrc_t x, uint32_t cols, uint32_t batch,
-                                              uint32_t lane, Partial<BT>& p, const uint4 (&early)[2]) {
+                                              const RowSpan& rs, const Activations<BT>& x, uint32_t cols,
+                                              uint32_t lane, Partial<BT>& p, uint4 (&early)[early_rounds<BT>()][BT]) {
     using G = Geometry<ES>;
-    constexpr uint32_t V = G::V;
+    constexpr uint32_t V = G::V, kSpan = NZ_WAVE * V;   // elements per round
+    constexpr uint32_t E = early_rounds<BT>();
+    uint4 late[BT == 1 ? G::kRounds - E : 1][BT];   // one row: every later round; more: the odd rounds in turn
+    if (BT == 1) fetch_x<ES, BT, E, G::kRounds>(x, rs, ti, cols, lane, late);
 #pragma unroll
-    for (int b = 0; b < BT; ++b) {
-        // the activations of every round first (row 0's first two rounds were
-        // requested before the decode), then one round's weights at a time
-        uint4 xv[G::kRounds];
-#pragma unroll
-        for (uint32_t r = 0; r < G::kRounds; ++r) {
-            if (b == 0 && r < 2) {
-                xv[r] = early[r];
-                continue;
-            }
-            const uint32_t g = (lane + NZ_WAVE * r) * V;
-            const bool whole = g >= ti.s0 && g + V <= ti.s1;
-            const uint32_t col = rs.col0 + g - (g >= rs.split ? cols : 0u);
-            xv[r] = load_vector(x, whole && b < static_cast<int>(batch) ? (b * cols + col) * ES : kOutOfRange);
+    for (uint32_t r = 0; r < G::kRounds; ++r) {
+        if (ti.s1 <= r * kSpan) continue;
+        if (BT > 1 && r + 1 < G::kRounds) fetch_x_round<ES, BT>(x, rs, ti, cols, lane, r + 1, r % 2 ? early[0] : late[0]);
+        const uint4* xv = BT == 1 ? (r < E ? early[r % E] : late[(r - E) % (G::kRounds - E)]) : r % 2 ? late[0] : early[0];
+        const uint32_t g = (lane + NZ_WAVE * r) * V;
+        const uint8_t* at = stage + NZ_STAGE_ORIGIN + g;
+        uint32_t e0, e1 = 0;
+        if (ES == 2) {
+            const uint2 e = *reinterpret_cast<const uint2*>(at);
+            e0 = e.x;
+            e1 = e.y;
+        } else {
+            e0 = *reinterpret_cast<const uint32_t*>(at);
         }
+        const uint4 v = merge_vector<ES, REORDER>(e0, e1, d.raw[r]);
+        if (ti.s0 == 0 && min(ti.s1, rs.split) >= (r + 1) * kSpan) {   // every vector inside the tile's first row
+            asm volatile("");
 #pragma unroll
-        for (uint32_t r = 0; r < G::kRounds; ++r) {
-            const uint32_t g = (lane + NZ_WAVE * r) * V;
-            const bool whole = g >= ti.s0 && g + V <= ti.s1;
-            const uint8_t* at = stage + NZ_STAGE_ORIGIN + (whole ? g : 0u);
-            uint32_t e0, e1 = 0;
-            if (ES == 2) {
-                const uint2 e = *reinterpret_cast<const uint2*>(at);
-                e0 = e.x;
-                e1 = e.y;
-            } else {
-                e0 = *reinterpret_cast<const uint32_t*>(at);
+            for (int b = 0; b < BT; ++b) p.acc[0][b] = dot_vector<ES, REORDER>(v, xv[b], p.acc[0][b]);
+        } else {
+            asm volatile("");
+            // staged bytes outside the tile are the neighbours': keep them out of the sums
+            // (the round's first element on the scalar side of the comparisons)
+            const int32_t v0 = static_cast<int32_t>(lane * V);
+            const bool whole = g >= ti.s0 && v0 <= static_cast<int32_t>(ti.s1 - V - r * kSpan);
+            const bool hi = v0 >= static_cast<int32_t>(rs.split - r * kSpan);
+#pragma unroll
+            for (int b = 0; b < BT; ++b) {
+                const float dot = dot_vector<ES, REORDER>(v, xv[b], 0.0f);
+                p.acc[0][b] += whole && !hi ? dot : 0.0f;
+                p.acc[1][b] += whole && hi ? dot : 0.0f;
             }
-            const uint4 v = merge_vector<ES, REORDER>(e0, e1, d.raw[r]);
-            // staged bytes outside the tile are stale: keep them out of the sums
-            const float dot = whole ? dot_vector<ES, REORDER>(v, xv[r], 0.0f) : 0.0f;
-            const bool hi = g >= rs.split;
-            p.acc[0][b] += hi ? 0.0f : dot;
-            p.acc[1][b] += hi ? dot : 0.0f;
         }
     }
     if (ti.s0 != 0 || ti.s1 % V != 0) {   // elements of the partial first and last vectors (fragment ends)
@@ -216,15 +274,14 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
         const bool partial = !(vec0 >= ti.s0 && vec0 + V <= ti.s1);
         const bool mine = lane < 2 * V && (lane < V || ti.nv > 1) && partial && g >= ti.s0 && g < ti.s1;
         const uint32_t expo = stage[NZ_STAGE_ORIGIN + (mine ? g : 0u)];
-        const float wf = mine ? word_to_float<ES, REORDER>(restore_word<ES, REORDER>((expo << (8 * (ES - 1))) | d.edge))
+        const float wf = mine ? word_to_float<ES, REORDER>(element_word<ES, REORDER>(expo, d.edge))
                               : 0.0f;
         const bool h = g >= rs.split;
-        const uint32_t col = rs.col0 + g - (h ? cols : 0u);
+        const uint32_t off = mine ? (rs.col0 + g - (h ? cols : 0u)) * ES : kOutOfRange;
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
-            const uint32_t off = mine && b < static_cast<int>(batch) ? (b * cols + col) * ES : kOutOfRange;
-            const uint32_t xw = ES == 2 ? __builtin_amdgcn_raw_buffer_load_b16(x, off, 0, 0)
-                                        : __builtin_amdgcn_raw_buffer_load_b32(x, off, 0, 0);
+            const uint32_t xw = ES == 2 ? __builtin_amdgcn_raw_buffer_load_b16(x.row[b], off, 0, 0)
+                                        : __builtin_amdgcn_raw_buffer_load_b32(x.row[b], off, 0, 0);
             const float prod = wf * word_to_float<ES, REORDER>(xw);
             p.acc[0][b] += h ? 0.0f : prod;
             p.acc[1][b] += h ? prod : 0.0f;
@@ -236,9 +293,10 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
 template <int ES, bool REORDER, bool LONG, bool ESC, int BT>
 __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_matvec_tile* tiles, const nz_work& seg,
                                                 uint32_t* counter, uint32_t lane, const uint32_t* lut, uint8_t* stage,
-                                                uint32_t cols, rsrc_t x, uint32_t batch, rsrc_t partials) {
+                                                uint32_t cols, const Activations<BT>& x, uint32_t batch,
+                                                float* partials) {
     const uint32_t n = seg.tile1 - seg.tile0;
-    uint32_t t = claim(counter, lane);
+    uint32_t t = claim(counter);
     if (t >= n) return;
     // The next tile's windows are requested a tile ahead; this tile's raw
     // lanes and its first activations at its start, so that the decode hides
@@ -248,27 +306,22 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
     TileInfo cur = tile_record<ES>(base, tiles, seg.tile0 + t, cols, rs);
     Fetch<ES, LONG> fc;
     fetch_bits<ES, LONG>(cur, lane, fc);
-    uint32_t tn = claim(counter, lane);
+    uint32_t tn = claim(counter);
     Partial<BT> p;
     for (;;) {
         const bool more = tn < n;
         RowSpan rn;
         const TileInfo nxt = tile_record<ES>(base, tiles, seg.tile0 + (more ? tn : t), cols, rn);
         Fetch<ES, LONG> fn;
-        fetch_bits<ES, LONG>(nxt, lane, fn);
-        const uint32_t after = more ? claim(counter, lane) : n;
+        const uint32_t after = more ? claim(counter) : n;
         fetch_raw<ES, LONG>(cur, lane, fc);
-        uint4 early[2];   // activation row 0 of rounds 0 and 1
-#pragma unroll
-        for (uint32_t r = 0; r < 2; ++r) {
-            const uint32_t g = (lane + NZ_WAVE * r) * Geometry<ES>::V;
-            const bool whole = g >= cur.s0 && g + Geometry<ES>::V <= cur.s1;
-            const uint32_t col = rs.col0 + g - (g >= rs.split ? cols : 0u);
-            early[r] = load_vector(x, whole ? col * ES : kOutOfRange);
-        }
-        stage_tile<ES, LONG, ESC>(cur, fc, lut, stage, lane);
+        uint4 early[early_rounds<BT>()][BT];
+        fetch_x<ES, BT, 0, early_rounds<BT>()>(x, rs, cur, cols, lane, early);
+        const LaneDecode l = open_tile<ES, LONG>(cur, fc, stage, lane);
+        fetch_bits<ES, LONG>(nxt, lane, fn);   // into the registers the open tile no longer needs
+        decode_tile<LONG, ESC>(l, lut);
         p.clear();
-        multiply_tile<ES, REORDER, LONG, BT>(cur, fc, stage, rs, x, cols, batch, lane, p, early);
+        multiply_tile<ES, REORDER, LONG, BT>(cur, fc, stage, rs, x, cols, lane, p, early);
         p.flush(partials, rs, rs.split < cur.s1, batch, lane);
         if (!more) break;
         t = tn;
@@ -282,7 +335,7 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
 // A raw (uncoded) tile: the exponent lane is stored as is.
 template <int ES, bool REORDER, int BT>
 __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_matvec_tile* tiles, uint32_t t, uint32_t cols,
-                         rsrc_t x, uint32_t batch, uint32_t lane, Partial<BT>& p, RowSpan& rs, bool& two) {
+                         const Activations<BT>& x, uint32_t lane, Partial<BT>& p, RowSpan& rs, bool& two) {
     constexpr uint32_t V = 16 / ES;
     const TileInfo ti = tile_record<ES>(base, tiles, t, cols, rs);
     two = rs.split < ti.s1;
@@ -306,12 +359,12 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_matvec_tile*
                 r[1] = *reinterpret_cast<const uint32_t*>(lanes + stride);
                 r[2] = *reinterpret_cast<const uint32_t*>(lanes + 2 * stride);
             }
-            const uint4 w = merge_vector<ES, REORDER>(e0, e1, r);
+            const uint4 w = merge_vector<ES, REORDER>(staged_form<REORDER>(e0), staged_form<REORDER>(e1), r);
             const bool h = g >= rs.split;
             const uint32_t col = rs.col0 + g - (h ? cols : 0u);
 #pragma unroll
             for (int b = 0; b < BT; ++b) {
-                const uint4 xv = load_vector(x, b < static_cast<int>(batch) ? (b * cols + col) * ES : kOutOfRange);
+                const uint4 xv = load_vector(x.row[b], col * ES);
                 const float dot = dot_vector<ES, REORDER>(w, xv, 0.0f);
                 p.acc[0][b] += h ? 0.0f : dot;
                 p.acc[1][b] += h ? dot : 0.0f;
@@ -327,9 +380,8 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_matvec_tile*
                 const uint32_t col = rs.col0 + g + j - (h ? cols : 0u);
 #pragma unroll
                 for (int b = 0; b < BT; ++b) {
-                    const uint32_t off = b < static_cast<int>(batch) ? (b * cols + col) * ES : kOutOfRange;
-                    const uint32_t xw = ES == 2 ? __builtin_amdgcn_raw_buffer_load_b16(x, off, 0, 0)
-                                                : __builtin_amdgcn_raw_buffer_load_b32(x, off, 0, 0);
+                    const uint32_t xw = ES == 2 ? __builtin_amdgcn_raw_buffer_load_b16(x.row[b], col * ES, 0, 0)
+                                                : __builtin_amdgcn_raw_buffer_load_b32(x.row[b], col * ES, 0, 0);
                     const float prod = wf * word_to_float<ES, REORDER>(xw);
                     p.acc[0][b] += h ? 0.0f : prod;
                     p.acc[1][b] += h ? prod : 0.0f;
@@ -340,50 +392,41 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_matvec_tile*
 }
 
 template <int ES, bool REORDER, bool LONG, int BT>
-__global__ __launch_bounds__(matvec_threads<BT>()) __attribute__((amdgpu_waves_per_eu(BT == 1 ? 8 : 6)))
+__global__ __launch_bounds__(matvec_threads<BT>()) __attribute__((amdgpu_waves_per_eu(BT <= 2 ? 8 : 6)))
 void nz_matvec_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __restrict__ frags,
                       const nz_matvec_tile* __restrict__ tiles, const nz_work* __restrict__ segs, uint32_t cols,
-                      const uint8_t* __restrict__ xp, uint32_t batch, float* __restrict__ partials_p, uint32_t n_tiles) {
-    using G = Geometry<ES>;
-    __shared__ __align__(16) uint32_t s_lut[NZ_LUT_MAX_WORDS];
-    __shared__ __align__(16) uint8_t s_stage[matvec_waves<BT>()][G::kStage];
-    __shared__ uint32_t s_claim;
+                      const uint8_t* __restrict__ xp, uint32_t batch, float* __restrict__ partials) {
+    __shared__ __align__(16) GroupLds<ES, matvec_waves<BT>()> lds;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NZ_WAVE);
-    const uint32_t lane = threadIdx.x % NZ_WAVE;
+    const uint32_t lane = lane_index();
     const nz_work seg = segs[blockIdx.x];
-    const rsrc_t x = make_rsrc(xp, batch * cols * ES);
-    const rsrc_t partials = make_rsrc(partials_p, n_tiles * 2u * batch * 4u);
-    if (threadIdx.x == 0) s_claim = 0;
+    const Activations<BT> x = activations<ES, BT>(xp, cols, batch);
+    if (threadIdx.x == 0) lds.claim[0] = 0;
     if (seg.kind == NZ_KIND_RAW) {
         __syncthreads();
         const uint32_t n = seg.tile1 - seg.tile0;
         Partial<BT> p;
-        for (uint32_t t = claim(&s_claim, lane); t < n; t = claim(&s_claim, lane)) {
+        for (uint32_t t = claim(lds.claim); t < n; t = claim(lds.claim)) {
             p.clear();
             RowSpan rs;
             bool two;
-            raw_tile<ES, REORDER, BT>(base, tiles, seg.tile0 + t, cols, x, batch, lane, p, rs, two);
+            raw_tile<ES, REORDER, BT>(base, tiles, seg.tile0 + t, cols, x, lane, p, rs, two);
             p.flush(partials, rs, two, batch, lane);
         }
         return;
     }
-    const uint4* img = reinterpret_cast<const uint4*>(base + frags[seg.lut_frag].lut);
-    // the host checks every image against NZ_LUT_MAX_WORDS; the clamp keeps a
-    // malformed one from overwriting the staging areas behind s_lut
-    const uint32_t words = min(reinterpret_cast<const uint32_t*>(img)[2], uint32_t(NZ_LUT_MAX_WORDS));
-    uint4* dst = reinterpret_cast<uint4*>(s_lut);
-    for (uint32_t i = threadIdx.x; i < (words + 3) / 4; i += matvec_threads<BT>()) dst[i] = img[i];
+    load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
     __syncthreads();
     if constexpr (LONG) {
-        huffman_segment<ES, REORDER, true, true, BT>(base, tiles, seg, &s_claim, lane, s_lut, s_stage[wave], cols,
+        huffman_segment<ES, REORDER, true, true, BT>(base, tiles, seg, lds.claim, lane, lds.lut, lds.stage[wave], cols,
                                                      x, batch, partials);
     } else {
-        if (s_lut[0])
-            huffman_segment<ES, REORDER, false, true, BT>(base, tiles, seg, &s_claim, lane, s_lut,
-                                                          s_stage[wave], cols, x, batch, partials);
+        if (lds.lut[0])
+            huffman_segment<ES, REORDER, false, true, BT>(base, tiles, seg, lds.claim, lane, lds.lut,
+                                                          lds.stage[wave], cols, x, batch, partials);
         else
-            huffman_segment<ES, REORDER, false, false, BT>(base, tiles, seg, &s_claim, lane, s_lut,
-                                                           s_stage[wave], cols, x, batch, partials);
+            huffman_segment<ES, REORDER, false, false, BT>(base, tiles, seg, lds.claim, lane, lds.lut,
+                                                           lds.stage[wave], cols, x, batch, partials);
     }
 }
 
@@ -454,7 +497,7 @@ hipError_t launch_matvec(const void* base, const void* frags, const void* tiles,
     hipLaunchKernelGGL((nz_matvec_kernel<ES, REORDER, LONG, BT>), dim3(n_segs), dim3(matvec_threads<BT>()), 0, stream,
                        static_cast<const uint8_t*>(base), static_cast<const nz_frag_desc*>(frags),
                        static_cast<const nz_matvec_tile*>(tiles), static_cast<const nz_work*>(segs), cols,
-                       static_cast<const uint8_t*>(x), batch, partials, n_tiles);
+                       static_cast<const uint8_t*>(x), batch, partials);
     return hipGetLastError();
 }
 

@@ -16,7 +16,7 @@
 
 namespace {
 
-constexpr int kIcmpUlt = 36;   // unsigned-less-than predicate of the lane-mask compare builtin
+constexpr int kIcmpUge = 35, kIcmpUlt = 36;   // unsigned predicates of the lane-mask compare builtin
 // s_waitcnt operand (gfx9 encoding) that waits for every outstanding LDS
 // operation: lgkmcnt 0, vmcnt 63 and expcnt 7 (no wait on those).
 constexpr int kWaitLgkm0 = 0xC07F;
@@ -67,22 +67,24 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // Canonical decode of one code longer than 12 bits whose prefix holds codes
-// of several lengths: from record `k` on, find the first escape length whose
-// left-justified limit exceeds the window. Returns the escape token entry;
-// *len receives the code length.
-__device__ __forceinline__ uint32_t escape_search(const uint32_t* lut, uint64_t window, uint32_t k, uint32_t* len) {
-    const uint32_t n_len = lut[0];
-    const uint32_t* rec = lut + NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES;
-    while (k + 1 < n_len) {
-        const uint64_t limit = rec[NZ_ESC_RECORD * k] | (static_cast<uint64_t>(rec[NZ_ESC_RECORD * k + 1]) << 32);
-        if (window < limit) break;
-        ++k;
-    }
-    const uint32_t* r = rec + NZ_ESC_RECORD * k;
-    const uint64_t first = r[2] | (static_cast<uint64_t>(r[3]) << 32);
-    const uint32_t L = r[5];
+// of three or more lengths, or longer than 32 bits: from record `k` on, find
+// the first escape length whose left-justified limit exceeds the window.
+// Returns the image word of the code's token; *len receives its length.
+// Without LONG all codes end within the window's first 32 bits.
+template <bool LONG>
+__device__ __forceinline__ uint32_t escape_search(const uint32_t* lut, uint32_t w0, uint32_t w1, uint32_t k,
+                                                  uint32_t* len) {
+    const uint32_t records = NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES, tokens = records + NZ_ESC_RECORD * lut[0];
+    uint32_t r = records + NZ_ESC_RECORD * k;
+    const uint64_t window = (static_cast<uint64_t>(w0) << 32) | w1;
+    for (; r + NZ_ESC_RECORD < tokens; r += NZ_ESC_RECORD)
+        if (LONG ? window < (lut[r] | (static_cast<uint64_t>(lut[r + 1]) << 32)) : w0 < lut[r + 1]) break;
+    const uint32_t L = lut[r + 5];
     *len = L;
-    return rec[NZ_ESC_RECORD * n_len + r[4] + static_cast<uint32_t>((window - first) >> (64 - L))];
+    const uint32_t offset =
+        LONG ? static_cast<uint32_t>((window - (lut[r + 2] | (static_cast<uint64_t>(lut[r + 3]) << 32))) >> (64 - L))
+             : (w0 - lut[r + 3]) >> (32 - L);
+    return tokens + lut[r + 4] + offset;
 }
 
 template <int ES, bool REORDER>
@@ -93,21 +95,39 @@ __device__ __forceinline__ uint32_t restore_word(uint32_t v) {
     return (v & 0x007FFFFFu) | ((v << 8) & 0x80000000u) | ((v >> 1) & 0x7F800000u);
 }
 
-// Four elements' top two bytes from four exponent bytes `e` and the four
-// stored bytes below them `r` (bit 7 = sign when reordered): returns the
+// Staged form of exponent bytes: with REORDER each byte is rotated right by
+// one bit, so that exponent >> 1 and the exponent's lowest bit sit where the
+// restored bytes hold them and merging takes one bit-field insert per dword
+// instead of a shift and an insert (8 of a 16-byte vector's 20 vector
+// instructions before). The LUT's copy in LDS holds its bytes in this form.
+template <bool REORDER>
+__device__ __forceinline__ uint32_t staged_form(uint32_t e) {
+    return REORDER ? bfi(0x7F7F7F7Fu, e >> 1, e << 7) : e;
+}
+
+// One element's word from its staged exponent byte and its raw lane bytes
+// `raw` (lane k in byte k).
+template <int ES, bool REORDER>
+__device__ __forceinline__ uint32_t element_word(uint32_t staged, uint32_t raw) {
+    const uint32_t expo = REORDER ? ((staged << 1) | (staged >> 7)) & 0xFFu : staged;
+    return restore_word<ES, REORDER>((expo << (8 * (ES - 1))) | raw);
+}
+
+// Four elements' top two bytes from four staged exponent bytes `e` and the
+// four stored bytes below them `r` (bit 7 = sign when reordered): returns the
 // restored high bytes in *hi and the bytes below them in *lo.
 template <bool REORDER>
 __device__ __forceinline__ void restore_pairs(uint32_t e, uint32_t r, uint32_t* hi, uint32_t* lo) {
     if (REORDER) {
-        *hi = bfi(0x7F7F7F7Fu, e >> 1, r);    // sign | exponent >> 1
-        *lo = bfi(0x7F7F7F7Fu, r, e << 7);    // exponent bit 0 | low mantissa bits
+        *hi = bfi(0x7F7F7F7Fu, e, r);    // sign | exponent >> 1
+        *lo = bfi(0x7F7F7F7Fu, r, e);    // exponent bit 0 | low mantissa bits
     } else {
         *hi = e;
         *lo = r;
     }
 }
 
-// A whole 16-byte vector of V elements. `e` holds V exponent bytes (two
+// A whole 16-byte vector of V elements. `e` holds V staged exponent bytes (two
 // dwords for 2-byte words, one for 4-byte words); `r` the raw lane dwords
 // (lane 0 for 2-byte words; lanes 0, 1, 2 for 4-byte words).
 template <int ES, bool REORDER>
@@ -248,12 +268,6 @@ __device__ __forceinline__ void fetch_raw(const TileInfo& ti, uint32_t lane, Fet
     }
 }
 
-template <int ES, bool LONG>
-__device__ __forceinline__ void fetch(const TileInfo& ti, uint32_t lane, Fetch<ES, LONG>& d) {
-    fetch_bits<ES, LONG>(ti, lane, d);
-    fetch_raw<ES, LONG>(ti, lane, d);
-}
-
 __device__ __forceinline__ uint2 lut_entry(const uint32_t* lut, uint32_t w0) {
     return reinterpret_cast<const uint2*>(lut + NZ_LUT_HEADER)[w0 >> (32 - NZ_LUT_BITS)];
 }
@@ -265,103 +279,133 @@ __device__ __forceinline__ uint2 lut_entry(const uint32_t* lut, uint32_t w0) {
 template <bool LONG, bool ESC>
 __device__ __forceinline__ uint2 lut_step(const uint32_t* lut, uint2 e, uint32_t& w0, uint32_t& w1, uint32_t& w2,
                                           uint32_t& w3) {
-    uint32_t s = e.x;   // the funnel shift reads its low five bits
     if (ESC) {
-        // One scalar branch where no lane escapes (0.5 % of a lane's steps
-        // do, so three steps in ten of a wavefront); the empty asm keeps the
-        // compiler from folding the lanes' test into it. An escape entry
-        // names the token of almost every escape, one LDS read: searching
-        // the length records for each one took 35 % of the fused kernel's
-        // vector instructions and 65 % of its scalar ones (58.7 M bf16
-        // elements, 59.2 -> 51.0 us for the product).
+        // One scalar branch where no lane escapes (0.8 % of a lane's steps
+        // do, so three steps in ten of a wavefront), and inside it one more
+        // where all lanes' codes have their prefix's first length; the empty
+        // asm keeps the compiler from folding the lanes' tests into them. An
+        // escape entry names the token of almost every escape, one LDS read:
+        // searching the length records for each one took 35 % of the fused
+        // kernel's vector instructions and 65 % of its scalar ones.
         if (__builtin_expect(__builtin_amdgcn_uicmp(e.x, 1u << NZ_ENTRY_COUNT, kIcmpUlt) != 0, 0)) {
             asm volatile("");
             if (e.x < (1u << NZ_ENTRY_COUNT)) {
-                if (e.x < NZ_ESC_SEARCH) {
-                    // the code's bits past the prefix count up from the prefix's first token
-                    e.x = lut[e.y + ((w0 << NZ_LUT_BITS) >> (NZ_LUT_BITS + s))];
-                } else {
-                    uint32_t len;
-                    e.x = escape_search(lut, (static_cast<uint64_t>(w0) << 32) | w1, e.y, &len);
-                    if (LONG && len > 32) {
-                        w0 = w1;
-                        w1 = w2;
-                        w2 = w3;
-                        w3 = 0;
-                        len -= 32;
+                // codes of one length under the prefix count up from its first token
+                const uint32_t rest = w0 << NZ_LUT_BITS, n = e.x >> NZ_ESC_COUNT;
+                uint32_t token = e.y + (rest >> (e.x & 31u)), s = e.x - NZ_LUT_BITS;
+                if (__builtin_expect(__builtin_amdgcn_uicmp(rest >> (e.x & 31u), n, kIcmpUge) != 0, 0)) {
+                    asm volatile("");
+                    if (e.x == NZ_ESC_SEARCH) {
+                        uint32_t len;
+                        token = escape_search<LONG>(lut, w0, w1, e.y, &len);
+                        if (LONG && len > 32) {
+                            w0 = w1;
+                            w1 = w2;
+                            w2 = w3;
+                            w3 = 0;
+                            len -= 32;
+                        }
+                        s = 32 - len;   // len in [1, 32]; s == 0 shifts a whole word
+                    } else if (rest >> (e.x & 31u) >= n) {   // the prefix's second length
+                        s = (e.x >> NZ_ESC_SECOND) & 31u;
+                        token = e.y + n + (rest >> s) - (n << ((e.x & 31u) - s));
+                        s -= NZ_LUT_BITS;
                     }
-                    s = 32 - len;   // len in [1, 32]; s == 0 shifts a whole word
                 }
-                e.y = e.x & 0xFFFFu;   // one or two bytes
+                const uint32_t t = lut[token];
+                e.y = t & 0xFFFFu;   // one or two bytes
+                e.x = bfi(31u, s, t & ~0xFFFFu);
             }
         }
     }
-    w0 = funnel(w0, w1, s);
-    w1 = funnel(w1, w2, s);
-    w2 = funnel(w2, LONG ? w3 : 0u, s);
-    if (LONG) w3 = funnel(w3, 0u, s);
+    // the funnel shift reads its low five bits
+    w0 = funnel(w0, w1, e.x);
+    w1 = funnel(w1, w2, e.x);
+    w2 = funnel(w2, LONG ? w3 : 0u, e.x);
+    if (LONG) w3 = funnel(w3, 0u, e.x);
     return e;
 }
 
-// Decodes a tile's exponent bytes into the wavefront's staging area: staging
-// index i (from NZ_STAGE_ORIGIN) holds the byte of the element at workspace
-// index ti.first + i, for i in [ti.s0, ti.s1). Ends with the wavefront's LDS
-// writes visible to all of its lanes.
-//
-// The staging area is cleared first, and every write into it is an LDS
-// atomic OR of whole aligned dwords, so lanes may share a dword without any
-// ordering between them. A lane's bytes go to [at, at + count); its final
-// LUT step may emit up to three bytes past the count, and those are the next
-// window's first bytes (the bitstream is continuous: decoding on past a
-// window's last code decodes the codes that start in the next window), or,
-// after the tile's last window, bytes that no one reads. An OR therefore
-// only ever adds a byte's own value or zeros.
-template <int ES, bool LONG, bool ESC>
-__device__ __forceinline__ void stage_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, const uint32_t* lut,
-                                           uint8_t* stage, uint32_t lane) {
+// A lane's place in a tile's decode: its window, left-justified at the next
+// code, and its place in the staging area as -8 x the LDS byte address of its
+// next byte (`neg`) and of the byte after its last one (`stop`).
+struct LaneDecode {
+    uint32_t w0, w1, w2, w3;
+    uint32_t neg, stop;
+};
+
+// Clears the tile's staging bytes and sets up the decode of a tile from
+// its metadata and windows in `d`, which are free for the next tile after it.
+template <int ES, bool LONG>
+__device__ __forceinline__ LaneDecode open_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, uint8_t* stage,
+                                                uint32_t lane) {
     using G = Geometry<ES>;
-    constexpr uint32_t kUnits = G::kStage / 16;
-    static_assert(G::kStage % 16 == 0, "the staging area is cleared in 16-byte units");
+    // what the merge reads: the rounds that hold elements of the tile
 #pragma unroll
-    for (uint32_t u = lane; u < (kUnits + NZ_WAVE - 1) / NZ_WAVE * NZ_WAVE; u += NZ_WAVE)
-        if (u < kUnits) reinterpret_cast<uint4*>(stage)[u] = make_uint4(0u, 0u, 0u, 0u);
-    const uint32_t count = lane < ti.n_win ? d.meta >> 8 : 0u;
+    for (uint32_t r = 0; r < G::kCapacity / (8 * NZ_WAVE); ++r)
+        if (r < 2 || ti.s1 > 2 * 8 * NZ_WAVE)
+            *reinterpret_cast<uint2*>(stage + NZ_STAGE_ORIGIN + 8 * (lane + NZ_WAVE * r)) = make_uint2(0u, 0u);
+    const uint32_t count = d.meta >> 8;   // 0 past the tile's windows: their metadata loads are out of range
     // The first window's skipped bytes land in the staging area's prefix
-    // (NZ_STAGE_ORIGIN exceeds any skip, so the index stays positive).
-    const uint32_t at = NZ_STAGE_ORIGIN + ti.s0 + (wave_inclusive_scan(count) - count) - ti.skip;
-    if (count) {
-        uint32_t w0 = bswap32(d.w[0]), w1 = bswap32(d.w[1]), w2 = bswap32(d.w[2]), w3 = LONG ? bswap32(d.w[3]) : 0u;
-        {   // restart at the gap
-            uint32_t g = d.meta & 0xFFu;
-            if (LONG && g >= 32) { w0 = w1; w1 = w2; w2 = w3; w3 = 0; g -= 32; }
-            if (g) {
-                const uint32_t s = 32 - g;
-                w0 = funnel(w0, w1, s);
-                w1 = funnel(w1, w2, s);
-                w2 = funnel(w2, LONG ? w3 : 0u, s);
-                if (LONG) w3 = funnel(w3, 0u, s);
-            }
+    // (NZ_STAGE_ORIGIN exceeds any skip, so the address stays inside it).
+    const uint32_t base = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)stage));
+    const uint32_t end = base + NZ_STAGE_ORIGIN + ti.s0 - ti.skip + wave_inclusive_scan(count);
+    LaneDecode l;
+    l.stop = 0u - 8u * end;
+    l.neg = l.stop + 8u * count;
+    l.w0 = bswap32(d.w[0]), l.w1 = bswap32(d.w[1]), l.w2 = bswap32(d.w[2]), l.w3 = LONG ? bswap32(d.w[3]) : 0u;
+    uint32_t g = d.meta & 0xFFu;   // restart at the gap
+    if (LONG) {
+        if (g >= 32) { l.w0 = l.w1; l.w1 = l.w2; l.w2 = l.w3; l.w3 = 0; g -= 32; }
+        if (g) {
+            const uint32_t s = 32 - g;
+            l.w0 = funnel(l.w0, l.w1, s);
+            l.w1 = funnel(l.w1, l.w2, s);
+            l.w2 = funnel(l.w2, l.w3, s);
+            l.w3 = funnel(l.w3, 0u, s);
         }
-        // bit: 8 x the LDS byte address of the next byte (the staging area
-        // is 16-byte aligned, so bit & 31 is its place in its dword); LDS
-        // addresses stay below 2^17, so bit stays below 2^20
-        typedef __attribute__((address_space(3))) uint32_t lds_u32;
-        const uint32_t base = static_cast<uint32_t>(
-            reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)stage));
-        uint32_t bit = 8 * (base + at);
-        const uint32_t stop = bit + 8 * count;
-        // The next step's LUT read is issued before this step's ORs, so that
-        // its latency covers theirs; the last one's entry goes unused.
-        uint2 e = lut_entry(lut, w0);
+    } else {   // codes end within the window's 95 bits, so the gap is at most 31
+        const uint64_t high = ((static_cast<uint64_t>(l.w0) << 32) | l.w1) << g;
+        const uint64_t low = ((static_cast<uint64_t>(l.w1) << 32) | l.w2) << g;
+        l.w0 = static_cast<uint32_t>(high >> 32);
+        l.w1 = static_cast<uint32_t>(low >> 32);
+        l.w2 = static_cast<uint32_t>(low);
+    }
+    return l;
+}
+
+// Decodes a tile's exponent bytes into the wavefront's cleared staging area:
+// staging index i (from NZ_STAGE_ORIGIN) holds the staged exponent byte of the
+// element at workspace index ti.first + i, for i in [ti.s0, ti.s1). Ends with
+// the wavefront's LDS writes visible to all of its lanes.
+//
+// Every write into the area is an LDS atomic OR of whole aligned
+// dwords, so lanes may share a dword without any ordering between them. A
+// lane's bytes go to [neg, stop); its final LUT step may emit up to three
+// bytes past them, and those are the next window's first bytes (the bitstream
+// is continuous: decoding on past a window's last code decodes the codes that
+// start in the next window), or, after the tile's last window, bytes that no
+// one reads. An OR therefore only ever adds a byte's own value or zeros.
+template <bool LONG, bool ESC>
+__device__ __forceinline__ void decode_tile(LaneDecode l, const uint32_t* lut) {
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    if (l.neg > l.stop) {
+        uint2 e = lut_entry(lut, l.w0);
         do {
-            e = lut_step<LONG, ESC>(lut, e, w0, w1, w2, w3);
-            const uint2 next = lut_entry(lut, w0);
-            lds_u32* dst = (lds_u32*)(uintptr_t)((bit >> 3) & ~3u);
-            // The entry's bytes in this dword, and the ones past it: one
-            // 64-bit shift (two 32-bit shifts and a negation before).
-            const uint64_t both = static_cast<uint64_t>(e.y) << (bit & 31u);
-            const uint32_t low = static_cast<uint32_t>(both);
-            const uint32_t high = static_cast<uint32_t>(both >> 32);
+            e = lut_step<LONG, ESC>(lut, e, l.w0, l.w1, l.w2, l.w3);
+            // The entry's bytes go to [p, p + count): the dword of byte
+            // p - 1 and the one after it, so that two funnel shifts by
+            // 32 - 8 (p mod 4), zero for an aligned p, split them.
+            lds_u32* dst = (lds_u32*)(uintptr_t)static_cast<uint32_t>(~((static_cast<int32_t>(l.neg) >> 3) | 3));
+            const uint32_t low = funnel(e.y, 0u, l.neg), high = funnel(0u, e.y, l.neg);
+            l.neg -= e.x >> (NZ_ENTRY_COUNT - 3);   // 8 x the byte count (bits 26 and 25 of a step's entry are zero)
+            // The next step's LUT read is issued before this step's ORs, so
+            // that their latencies overlap; the last one's entry goes
+            // unused. Nothing is left for a register copy: all uses of the
+            // entry come before the read that replaces it.
+            __builtin_amdgcn_sched_barrier(0);
+            e = lut_entry(lut, l.w0);
             __hip_atomic_fetch_or(dst, low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             __hip_atomic_fetch_or(dst + 1, high, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             // The read and the ORs complete before the wavefront issues its
@@ -369,20 +413,59 @@ __device__ __forceinline__ void stage_tile(const TileInfo& ti, const Fetch<ES, L
             // same wavefront's LDS atomics were still in flight has returned
             // staging data in place of the LUT entry, now and then.
             __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-            bit += e.x >> (NZ_ENTRY_COUNT - 3);   // 8 x the byte count (bits 5-26 of an entry are zero)
-            e = next;
-        } while (bit < stop);
+        } while (l.neg > l.stop);
     }
     wave_lds_sync();
 }
 
-// The next tile index of the workgroup's segment for this wavefront (one LDS
-// atomic from lane 0, broadcast). Indices at or past the segment's size mean
-// it is used up.
-__device__ __forceinline__ uint32_t claim(uint32_t* counter, uint32_t lane) {
-    uint32_t v = 0;
-    if (lane == 0) v = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    return __builtin_amdgcn_readfirstlane(v);
+// Copies a segment's LUT image into LDS, its bytes in staged form.
+template <bool REORDER, int THREADS>
+__device__ __forceinline__ void load_lut(const uint8_t* image, uint32_t* lut, uint32_t thread) {
+    const uint4* img = reinterpret_cast<const uint4*>(image);
+    // the host checks every image against NZ_LUT_MAX_WORDS; the clamp keeps a
+    // malformed one from overwriting the staging areas behind the LUT
+    const uint32_t words = min(reinterpret_cast<const uint32_t*>(img)[2], uint32_t(NZ_LUT_MAX_WORDS));
+    const uint32_t tokens = NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * reinterpret_cast<const uint32_t*>(img)[0];
+    uint4* dst = reinterpret_cast<uint4*>(lut);
+    for (uint32_t i = thread; i < (words + 3) / 4; i += THREADS) {
+        uint4 v = img[i];
+        if (i >= 1 && i < 1 + NZ_LUT_ENTRIES / 2) {   // two primary entries
+            if (v.x >> NZ_ENTRY_COUNT) v.y = staged_form<REORDER>(v.y);
+            if (v.z >> NZ_ENTRY_COUNT) v.w = staged_form<REORDER>(v.w);
+        } else if (REORDER) {   // escape tokens: two bytes below the count
+            uint32_t* w = &v.x;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if (4 * i + k >= tokens) w[k] = bfi(0xFFFFu, staged_form<true>(w[k] & 0xFFFFu), w[k]);
+        }
+        dst[i] = v;
+    }
+}
+
+// A workgroup's LDS. The claim counter comes first: ds_append takes its
+// address from M0's low 16 bits, which reach the first 64 KB.
+template <int ES, int WAVES>
+struct GroupLds {
+    uint32_t claim[4];
+    uint32_t lut[(NZ_LUT_MAX_WORDS + 3) / 4 * 4];
+    uint8_t stage[WAVES][Geometry<ES>::kStage];
+};
+
+// This thread's lane. The compiler does not see its range, so it keeps
+// lane * size + constant as an address and an immediate offset instead of one
+// register per constant.
+__device__ __forceinline__ uint32_t lane_index() {
+    uint32_t lane = threadIdx.x % NZ_WAVE;
+    asm("" : "+v"(lane));
+    return lane;
+}
+
+// The next tile index of the workgroup's segment for this wavefront: one
+// ds_append, which adds the number of its active lanes (all 64) to the
+// counter. Indices at or past the segment's size mean it is used up.
+__device__ __forceinline__ uint32_t claim(uint32_t* counter) {
+    typedef __attribute__((address_space(3))) int lds_int;
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(__builtin_amdgcn_ds_append((lds_int*)counter))) / NZ_WAVE;
 }
 
 }  // namespace

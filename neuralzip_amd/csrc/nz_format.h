@@ -61,16 +61,22 @@
 // (SDWA) adds to a bit position; word 1 is stored as one dword.
 // Escape token entry: b0 | b1 << 8 | byte count << 27.
 // An escape's primary entry (byte count 0) saves the kernels the search of
-// the records: where all codes under the prefix have one length L <= 32,
-//   word 0: 32 - L      word 1: image word of the token of its first code
-// (the code's L - 12 bits past the prefix count up from there), else
+// the records. Where the codes under the prefix have at most two lengths
+// L1 < L2 <= 32, the first n of them L1 (NZ_ESC_ALL: all of them),
+//   word 0: 44 - L1 | (44 - L2) << 5 | n << 10
+//   word 1: image word of the token of the prefix's first code
+// (the code's bits past the prefix, an L - 12 bit number, count up from the
+// first code of their length), else
 //   word 0: NZ_ESC_SEARCH      word 1: the record the search starts at.
 #define NZ_LUT_HEADER 4
 #define NZ_ESC_RECORD 6
 #define NZ_ENTRY_SHIFT_MASK 31u
 #define NZ_ENTRY_COUNT 27
 #define NZ_ENTRY_MAX_BYTES 4
-#define NZ_ESC_SEARCH 64u
+#define NZ_ESC_SECOND 5
+#define NZ_ESC_COUNT 10
+#define NZ_ESC_ALL 0xFFFFu
+#define NZ_ESC_SEARCH 0u
 #define NZ_LUT_MAX_WORDS (NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * 56 + 512)
 
 enum nz_kind : uint32_t { NZ_KIND_RAW = 0, NZ_KIND_SHORT = 1, NZ_KIND_LONG = 2 };

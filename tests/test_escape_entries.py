@@ -10,7 +10,7 @@ from neuralzip_amd import _native
 from nz_helpers import segment_lengths, segment_tensor
 
 VOCAB = bytes((127, 127, 125, 126))
-PRIMARY, SEARCH = 4, 64     # first primary entry; word 0 of an entry that searches the records
+PRIMARY, SEARCH = 4, 0     # first primary entry; word 0 of an entry that searches the records
 
 
 def spread_lengths(short, long, top):
@@ -54,9 +54,12 @@ def entry_token(lut, window):
     whose primary entry is an escape."""
     x = window >> 52
     e0, e1 = int(lut[PRIMARY + 2 * x]), int(lut[PRIMARY + 2 * x + 1])
-    if e0 < SEARCH:
-        w0 = window >> 32
-        return e1 + (((w0 << 12) & 0xFFFFFFFF) >> (12 + e0)), 32 - e0
+    if e0 != SEARCH:
+        rest, n = (window >> 20) & 0xFFFFF000, e0 >> 10     # the 20 bits past the prefix, left-justified
+        first, second = e0 & 31, e0 >> 5 & 31
+        if rest >> first < n:
+            return e1 + (rest >> first), 44 - first
+        return e1 + n + (rest >> second) - (n << (first - second)), 44 - second
     n, records = int(lut[0]), lut[PRIMARY + 8192:].astype(np.uint64)
     k = e1
     while k + 1 < n and window >= int(records[6 * k]) | int(records[6 * k + 1]) << 32:
@@ -81,9 +84,9 @@ def test_every_escape_entry_leads_to_its_code(name):
             assert lut[PRIMARY + 2 * (window >> 52)] >> 27 == 0
             word, length = entry_token(lut, window)
             assert length == n and lut[word] == value | width << 27
-    if name.startswith("spread"):   # entries of both kinds
-        kinds = {int(lut[PRIMARY + 2 * x]) < SEARCH for x in range(4096) if lut[PRIMARY + 2 * x] >> 27 == 0}
-        assert kinds == {True, False}
+    if name == "spread-6-9-20":   # prefixes of one length, of two, and of more
+        entries = [int(lut[PRIMARY + 2 * x]) for x in range(4096) if lut[PRIMARY + 2 * x] >> 27 == 0]
+        assert {"search" if e == SEARCH else e >> 10 < 0xFFFF for e in entries} == {"search", True, False}
 
 
 @pytest.mark.gpu
