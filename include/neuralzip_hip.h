@@ -9,8 +9,8 @@
  *   - every buffer is caller-owned; the library never frees caller memory;
  *   - int results: 0 on success, a negative nz_status on failure, with a
  *     thread-local message from nz_last_error();
- *   - host functions are re-entrant; nz_decode_launch, nz_matvec_launch and
- *     nz_matvec_reduce are asynchronous and
+ *   - host functions are re-entrant; nz_decode_launch, nz_matvec_launch,
+ *     nz_matvec_reduce and nz_matvec_rows are asynchronous and
  *     ordered on the given HIP stream.
  */
 #ifndef NEURALZIP_HIP_H
@@ -44,6 +44,7 @@ typedef struct nz_frag_desc nz_frag_desc;   /* 64 bytes */
 typedef struct nz_tile nz_tile;             /* 16 bytes */
 typedef struct nz_work nz_work;             /* 16 bytes */
 typedef struct nz_matvec_tile nz_matvec_tile; /* 40 bytes */
+typedef struct nz_row_work nz_row_work;       /* 32 bytes */
 
 const char* nz_last_error(void);
 int nz_abi_version(void);
@@ -309,6 +310,36 @@ int nz_matvec_launch(const void* base, const nz_frag_desc* frags, const nz_matve
  * reference (see nz_matvec_plan). */
 int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights, uint32_t n_weights,
                      const float* partials, uint32_t batch, int element_size, int bit_reorder, void* stream);
+
+/* Plan of the same product for one launch without partial sums in device
+ * memory: segments (one workgroup each, 32 bytes, caller-allocated for
+ * `capacity`) whose workgroups own whole rows and add up their rows
+ * themselves. Tiles, weights, slots and first_weight as for nz_matvec_plan
+ * and nz_plan_work. *n_segments receives 0 where the product has no such
+ * plan: a row in tiles of two codebooks or of separate places of the launch
+ * order, or rows so long that whole rows would leave the workgroups
+ * unevenly loaded. words[i] (i = 0, 1, 2) receives the LDS words that the
+ * largest segment needs for up to 1, 2 and 4 activation rows; a launch
+ * takes at most nz_matvec_row_words. No counterpart in the reference (see
+ * nz_matvec_plan). */
+int nz_matvec_row_plan(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
+                       const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, int element_size,
+                       uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
+                       uint32_t* n_segments, uint32_t* words);
+
+/* LDS words one row segment may need at `batch` activation rows. */
+uint32_t nz_matvec_row_words(int element_size, uint32_t batch);
+
+/* The product over row segments of one codebook kind (long_codes), complete:
+ * weights[k].y as nz_matvec_launch and nz_matvec_reduce leave it, the same
+ * bits. `words`: the plan's for this batch, checked against
+ * nz_matvec_row_words. row_index is a device copy of nz_matvec_plan's.
+ * Asynchronous on `stream`. No counterpart in the reference (see
+ * nz_matvec_plan). */
+int nz_matvec_rows(const void* base, const nz_frag_desc* frags, const nz_matvec_tile* tiles,
+                   const nz_row_work* segments, uint32_t n_segments, uint32_t words, int element_size,
+                   int bit_reorder, int long_codes, const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
+                   const void* x, uint32_t batch, const uint32_t* row_index, void* stream);
 
 /* Bytes of partial sums the no-allocation product holds per GPU. */
 #define NZ_MATVEC_SCRATCH_BYTES (32u << 20)

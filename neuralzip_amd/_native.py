@@ -35,7 +35,10 @@ WORK = np.dtype([("tile0", "<u4"), ("tile1", "<u4"), ("lut_frag", "<u4"), ("kind
 # before the tile | lane stride << 4)
 MATVEC_TILE = np.dtype([("bits", "<u8"), ("meta", "<u8"), ("lanes", "<u8"), ("counts", "<u4"), ("head", "<u4"),
                         ("entry", "<u4"), ("col0", "<u4")])
+ROW_WORK = np.dtype([("tile0", "<u4"), ("tile1", "<u4"), ("lut_frag", "<u4"), ("kind", "<u4"), ("row0", "<u4"),
+                     ("row1", "<u4"), ("entry0", "<u4"), ("entries", "<u4")])
 assert FRAG_DESC.itemsize == 64 and TILE.itemsize == 16 and WORK.itemsize == 16 and MATVEC_TILE.itemsize == 40
+assert ROW_WORK.itemsize == 32
 
 KIND_RAW, KIND_SHORT, KIND_LONG = 0, 1, 2
 # Words of the kernels' LDS copy of a LUT image (NZ_LUT_MAX_WORDS of nz_format.h).
@@ -126,6 +129,12 @@ def lib():
         L.nz_matvec_launch.argtypes = [vp, vp, vp, vp, u32, ctypes.c_int, ctypes.c_int, ctypes.c_int, u32, vp, u32,
                                        vp, u32, vp]
         L.nz_matvec_reduce.argtypes = [vp, vp, u32, vp, u32, ctypes.c_int, ctypes.c_int, vp]
+        L.nz_matvec_row_plan.argtypes = [vp, vp, u32, vp, u32, u32, ctypes.c_int, u32, ctypes.c_double, vp, u32,
+                                         ctypes.POINTER(u32), vp]
+        L.nz_matvec_row_words.argtypes = [ctypes.c_int, u32]
+        L.nz_matvec_row_words.restype = u32
+        L.nz_matvec_rows.argtypes = [vp, vp, vp, vp, u32, u32, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, u32, u32,
+                                     vp, u32, vp, vp]
         L.nz_matvec_noalloc.argtypes = [vp, vp, vp, u32, vp, u32, vp, u32, ctypes.c_int, ctypes.c_int, vp, u32, u32,
                                         vp, u32, vp, vp]
         L.nz_chunk_histograms.argtypes = [vp, u64, ctypes.POINTER(_LaneLayout), u64, ctypes.c_int, vp, vp]
@@ -372,6 +381,19 @@ def matvec_tiles(descs, tiles, weights, cols, element_size, store_bytes):
                                 ctypes.cast(array, ctypes.c_void_p), len(weights), int(cols), int(element_size),
                                 int(store_bytes), out.ctypes.data if len(out) else None))
     return out
+
+
+def matvec_row_plan(descs, tiles, weights, cols, element_size, slots, first_weight=1.0):
+    """Row segments (ROW_WORK; empty where the product has none) and the LDS
+    words the largest one needs for up to 1, 2 and 4 activation rows."""
+    array = matvec_weights(weights)
+    rows = sum(int(w[1]) for w in weights)
+    out = np.zeros(min(rows, max(int(slots), len(tiles), 1)), dtype=ROW_WORK)   # a row or more per segment
+    n, words = ctypes.c_uint32(), (ctypes.c_uint32 * 3)()
+    check(lib().nz_matvec_row_plan(descs.ctypes.data, tiles.ctypes.data if len(tiles) else None, len(tiles),
+                                   ctypes.cast(array, ctypes.c_void_p), len(weights), int(cols), int(element_size),
+                                   int(slots), float(first_weight), out.ctypes.data, len(out), ctypes.byref(n), words))
+    return out[:n.value].copy(), tuple(words)
 
 
 def matvec_launch(base_ptr, frags_ptr, tiles_ptr, segments_ptr, n_segments, element_size, bit_reorder, long_codes,

@@ -48,6 +48,12 @@ extern "C" int nz_hip_matvec_launch(const void* base, const void* frags, const v
                                     uint32_t n_segs, int element_size, int bit_reorder, int long_codes, uint32_t cols,
                                     const void* x, uint32_t batch, float* partials, uint32_t n_tiles, void* stream,
                                     char* message, size_t message_size);
+extern "C" uint32_t nz_hip_matvec_row_words(int element_size, uint32_t batch);
+extern "C" int nz_hip_matvec_rows(const void* base, const void* frags, const void* tiles, const void* segs,
+                                  uint32_t n_segs, int element_size, int bit_reorder, int long_codes,
+                                  const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, const void* x,
+                                  uint32_t batch, const uint32_t* row_index, void* stream, char* message,
+                                  size_t message_size);
 extern "C" int nz_hip_matvec_noalloc(const void* base, const void* frags, const void* tiles, uint32_t n_tiles,
                                      const void* short_segs, uint32_t n_short, const void* long_segs,
                                      uint32_t n_long, int element_size, int bit_reorder,
@@ -353,6 +359,59 @@ int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights,
     char message[256] = {0};
     const int rc = nz_hip_matvec_reduce(row_index, weights, n_weights, partials, batch, element_size,
                                         bit_reorder, stream, message, sizeof message);
+    if (rc) return set_error(rc, message);
+    return 0;
+}
+
+int nz_matvec_row_plan(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
+                       const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, int element_size,
+                       uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
+                       uint32_t* n_segments, uint32_t* words) {
+    return guarded([&] {
+        if (!frags || (!tiles && n_tiles) || !weights || (!out && capacity) || !n_segments || !words)
+            nz::fail(nz::kInvalidArgument, "Null matvec plan argument.");
+        if (element_size != 2 && element_size != 4) nz::fail(nz::kInvalidArgument, "element_size must be 2 or 4.");
+        const std::vector<nz_row_work> segs =
+            nz::plan_rows(frags, tiles, n_tiles, weights, n_weights, cols, static_cast<unsigned>(element_size), slots,
+                          first_weight);
+        if (segs.size() > capacity) nz::fail(nz::kInvalidArgument, "Segment buffer is too small.");
+        std::copy(segs.begin(), segs.end(), out);
+        *n_segments = static_cast<uint32_t>(segs.size());
+        for (uint32_t i = 0; i < 3; ++i) {
+            uint64_t most = 0;
+            for (const nz_row_work& s : segs)
+                most = std::max<uint64_t>(most, s.row1 - s.row0 + 1ull + (static_cast<uint64_t>(s.entries) << i));
+            words[i] = static_cast<uint32_t>(std::min<uint64_t>(most, 0xFFFFFFFFull));
+        }
+    });
+}
+
+uint32_t nz_matvec_row_words(int element_size, uint32_t batch) { return nz_hip_matvec_row_words(element_size, batch); }
+
+int nz_matvec_rows(const void* base, const nz_frag_desc* frags, const nz_matvec_tile* tiles,
+                   const nz_row_work* segments, uint32_t n_segments, uint32_t words, int element_size,
+                   int bit_reorder, int long_codes, const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
+                   const void* x, uint32_t batch, const uint32_t* row_index, void* stream) {
+    if (!base || !frags || !tiles || !segments || !x || !weights || !row_index)
+        return set_error(nz::kInvalidArgument, "Null matvec argument.");
+    const int rc0 = guarded([&] {
+        if (element_size != 2 && element_size != 4) nz::fail(nz::kInvalidArgument, "element_size must be 2 or 4.");
+        if (n_weights == 0 || n_weights > NZ_MATVEC_MAX_WEIGHTS)
+            nz::fail(nz::kInvalidArgument, "A fused product takes 1 to 4 weights.");
+        if (!cols || cols % (16u / static_cast<unsigned>(element_size)))
+            nz::fail(nz::kInvalidArgument, "Row length must be a positive multiple of 16 bytes of elements.");
+        if (batch == 0 || batch > NZ_MATVEC_MAX_BATCH) nz::fail(nz::kInvalidArgument, "matvec batch must be in [1, 4].");
+        if (static_cast<uint64_t>(batch) * cols * static_cast<uint64_t>(element_size) > 0xFFFFFFFFull)
+            nz::fail(nz::kInvalidArgument, "Activation rows exceed the addressable range.");
+        if (words > nz_hip_matvec_row_words(element_size, batch))
+            nz::fail(nz::kLayoutLimit, "The plan's row segments exceed a workgroup's LDS at this batch.");
+        for (uint32_t k = 0; k < n_weights; ++k)
+            if (!weights[k].y) nz::fail(nz::kInvalidArgument, "Null matvec output.");
+    });
+    if (rc0) return rc0;
+    char message[256] = {0};
+    const int rc = nz_hip_matvec_rows(base, frags, tiles, segments, n_segments, element_size, bit_reorder, long_codes,
+                                      weights, n_weights, cols, x, batch, row_index, stream, message, sizeof message);
     if (rc) return set_error(rc, message);
     return 0;
 }

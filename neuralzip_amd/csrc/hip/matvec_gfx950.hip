@@ -16,11 +16,14 @@
 //     accumulated in fp32) and reduces its lanes with DPP. A tile holds at
 //     most 2048 elements, so with cols >= 2048 it touches at most two rows;
 //     the wavefront writes one partial sum per (row slot, activation row).
-//   * nz_matvec_reduce_kernel: one thread per output row adds the row's
+//   * nz_matvec_rows_kernel: the same for plans whose workgroups own whole
+//     rows, which add up their rows' partial sums in LDS: the whole product
+//     in one launch.
+//   * nz_matvec_reduce_kernel: otherwise, one thread per output row adds the row's
 //     partial sums, which sit at adjacent positions in element order (a
 //     host-built row index), adds the bias in fp32 and rounds once to the
 //     weight's dtype.
-// Both kernels fix the order of every addition, so repeated calls give
+// All of them fix the order of every addition, so repeated calls give
 // identical bits.
 #include <hip/hip_runtime.h>
 
@@ -138,6 +141,27 @@ __device__ __forceinline__ TileInfo tile_record(const uint8_t* base, const nz_ma
     return ti;
 }
 
+// Where partial sums go: the product's array in device memory, for the
+// reduce launch ...
+struct GlobalSums {
+    float* partials;
+    uint32_t batch;
+    __device__ __forceinline__ void put(uint32_t entry, int b, float v) const {
+        if (b < static_cast<int>(batch)) partials[entry * batch + b] = v;
+    }
+};
+
+// ... or, in a workgroup that owns whole rows, its LDS (positions of a
+// neighbour's rows, at the segment's ends, are left out).
+template <int BT>
+struct RowSums {
+    uint32_t* sums;
+    uint32_t entry0, entries;
+    __device__ __forceinline__ void put(uint32_t entry, int b, float v) const {
+        if (entry - entry0 < entries) sums[(entry - entry0) * BT + b] = __float_as_uint(v);
+    }
+};
+
 // The per-tile accumulators: acc[slot][b], slot 0 = row0, slot 1 = row0 + 1.
 template <int BT>
 struct Partial {
@@ -150,17 +174,16 @@ struct Partial {
     }
     // Reduces over the wavefront; lane 63 writes the tile's sums to partial
     // positions `entry` and, when the tile reaches the next row (`two`),
-    // entry + 1 (every other lane's stores fall outside the buffer range).
-    // Without `two`, position entry + 1 belongs to the next tile.
-    __device__ __forceinline__ void flush(float* __restrict__ partials, const RowSpan& rs, bool two, uint32_t batch,
-                                          uint32_t lane) {
+    // entry + 1. Without `two`, position entry + 1 belongs to the next tile.
+    template <class Sums>
+    __device__ __forceinline__ void flush(const Sums& sums, const RowSpan& rs, bool two, uint32_t lane) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int b = 0; b < BT; ++b) {
                 if (s == 1 && !two) break;
                 const float total = wave_sum(acc[s][b]);
-                if (lane == NZ_WAVE - 1 && b < static_cast<int>(batch)) partials[(rs.entry + s) * batch + b] = total;
+                if (lane == NZ_WAVE - 1) sums.put(rs.entry + s, b, total);
             }
     }
 };
@@ -290,12 +313,11 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
     wave_lds_sync();   // the staging area is rewritten by the next tile
 }
 
-template <int ES, bool REORDER, bool LONG, bool ESC, int BT>
-__device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_matvec_tile* tiles, const nz_work& seg,
+// One wavefront's share of a Huffman segment: `tiles` are the segment's n.
+template <int ES, bool REORDER, bool LONG, bool ESC, int BT, class Sums>
+__device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_matvec_tile* tiles, uint32_t n,
                                                 uint32_t* counter, uint32_t lane, const uint32_t* lut, uint8_t* stage,
-                                                uint32_t cols, const Activations<BT>& x, uint32_t batch,
-                                                float* partials) {
-    const uint32_t n = seg.tile1 - seg.tile0;
+                                                uint32_t cols, const Activations<BT>& x, const Sums& sums) {
     uint32_t t = claim(counter);
     if (t >= n) return;
     // The next tile's windows are requested a tile ahead; this tile's raw
@@ -303,7 +325,7 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
     // their latency (holding the next tile's raw lanes as well would not fit
     // the 64 registers of eight wavefronts per SIMD).
     RowSpan rs;
-    TileInfo cur = tile_record<ES>(base, tiles, seg.tile0 + t, cols, rs);
+    TileInfo cur = tile_record<ES>(base, tiles, t, cols, rs);
     Fetch<ES, LONG> fc;
     fetch_bits<ES, LONG>(cur, lane, fc);
     uint32_t tn = claim(counter);
@@ -311,7 +333,7 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
     for (;;) {
         const bool more = tn < n;
         RowSpan rn;
-        const TileInfo nxt = tile_record<ES>(base, tiles, seg.tile0 + (more ? tn : t), cols, rn);
+        const TileInfo nxt = tile_record<ES>(base, tiles, more ? tn : t, cols, rn);
         Fetch<ES, LONG> fn;
         const uint32_t after = more ? claim(counter) : n;
         fetch_raw<ES, LONG>(cur, lane, fc);
@@ -322,7 +344,7 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
         decode_tile<LONG, ESC>(l, lut);
         p.clear();
         multiply_tile<ES, REORDER, LONG, BT>(cur, fc, stage, rs, x, cols, lane, p, early);
-        p.flush(partials, rs, rs.split < cur.s1, batch, lane);
+        p.flush(sums, rs, rs.split < cur.s1, lane);
         if (!more) break;
         t = tn;
         tn = after;
@@ -391,43 +413,49 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_matvec_tile*
     }
 }
 
+// A workgroup's tiles, from its wavefronts' claims: `tiles` are the segment's n.
+template <int ES, bool REORDER, bool LONG, int BT, class Sums>
+__device__ __forceinline__ void run_segment(const uint8_t* base, const nz_matvec_tile* tiles, uint32_t n, uint32_t kind,
+                                            GroupLds<ES, matvec_waves<BT>()>& lds, uint32_t lane, uint32_t cols,
+                                            const Activations<BT>& x, const Sums& sums) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NZ_WAVE);
+    if (kind == NZ_KIND_RAW) {
+        Partial<BT> p;
+        for (uint32_t t = claim(lds.claim); t < n; t = claim(lds.claim)) {
+            p.clear();
+            RowSpan rs;
+            bool two;
+            raw_tile<ES, REORDER, BT>(base, tiles, t, cols, x, lane, p, rs, two);
+            p.flush(sums, rs, two, lane);
+        }
+    } else if constexpr (LONG) {
+        huffman_segment<ES, REORDER, true, true, BT>(base, tiles, n, lds.claim, lane, lds.lut, lds.stage[wave], cols, x,
+                                                     sums);
+    } else {
+        if (lds.lut[0])
+            huffman_segment<ES, REORDER, false, true, BT>(base, tiles, n, lds.claim, lane, lds.lut, lds.stage[wave],
+                                                          cols, x, sums);
+        else
+            huffman_segment<ES, REORDER, false, false, BT>(base, tiles, n, lds.claim, lane, lds.lut, lds.stage[wave],
+                                                           cols, x, sums);
+    }
+}
+
 template <int ES, bool REORDER, bool LONG, int BT>
 __global__ __launch_bounds__(matvec_threads<BT>()) __attribute__((amdgpu_waves_per_eu(BT <= 2 ? 8 : 6)))
 void nz_matvec_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __restrict__ frags,
                       const nz_matvec_tile* __restrict__ tiles, const nz_work* __restrict__ segs, uint32_t cols,
                       const uint8_t* __restrict__ xp, uint32_t batch, float* __restrict__ partials) {
     __shared__ __align__(16) GroupLds<ES, matvec_waves<BT>()> lds;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NZ_WAVE);
     const uint32_t lane = lane_index();
     const nz_work seg = segs[blockIdx.x];
     const Activations<BT> x = activations<ES, BT>(xp, cols, batch);
     if (threadIdx.x == 0) lds.claim[0] = 0;
-    if (seg.kind == NZ_KIND_RAW) {
-        __syncthreads();
-        const uint32_t n = seg.tile1 - seg.tile0;
-        Partial<BT> p;
-        for (uint32_t t = claim(lds.claim); t < n; t = claim(lds.claim)) {
-            p.clear();
-            RowSpan rs;
-            bool two;
-            raw_tile<ES, REORDER, BT>(base, tiles, seg.tile0 + t, cols, x, lane, p, rs, two);
-            p.flush(partials, rs, two, batch, lane);
-        }
-        return;
-    }
-    load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
+    if (seg.kind != NZ_KIND_RAW)
+        load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
     __syncthreads();
-    if constexpr (LONG) {
-        huffman_segment<ES, REORDER, true, true, BT>(base, tiles, seg, lds.claim, lane, lds.lut, lds.stage[wave], cols,
-                                                     x, batch, partials);
-    } else {
-        if (lds.lut[0])
-            huffman_segment<ES, REORDER, false, true, BT>(base, tiles, seg, lds.claim, lane, lds.lut,
-                                                          lds.stage[wave], cols, x, batch, partials);
-        else
-            huffman_segment<ES, REORDER, false, false, BT>(base, tiles, seg, lds.claim, lane, lds.lut,
-                                                           lds.stage[wave], cols, x, batch, partials);
-    }
+    run_segment<ES, REORDER, LONG, BT>(base, tiles + seg.tile0, seg.tile1 - seg.tile0, seg.kind, lds, lane, cols, x,
+                                       GlobalSums{partials, batch});
 }
 
 // fp32 to the weight's dtype, rounding to nearest even.
@@ -457,35 +485,106 @@ struct ReduceGroup {
     uint32_t total_rows;
 };
 
+// Which weight output row n of the stack belongs to.
+__device__ __forceinline__ uint32_t weight_of(const ReduceGroup& g, uint32_t n) {
+    uint32_t w = 0;
+#pragma unroll
+    for (uint32_t k = 1; k < NZ_MATVEC_MAX_WEIGHTS; ++k)
+        if (k < g.count && n >= g.row_base[k]) w = k;
+    return w;
+}
+
+// Weight w's bias for its row `local` in fp32, 0 without one.
+template <int ES, bool REORDER>
+__device__ __forceinline__ float row_bias(const ReduceGroup& g, uint32_t w, uint32_t local) {
+    const uint8_t* bias = g.bias[w];
+    return bias == nullptr ? 0.0f
+           : word_to_float<ES, REORDER>(ES == 2 ? reinterpret_cast<const uint16_t*>(bias)[local]
+                                                : reinterpret_cast<const uint32_t*>(bias)[local]);
+}
+
+// Sum of the values get(e0) .. get(e1 - 1) in that order, four reads in
+// flight at a time.
+template <class Get>
+__device__ __forceinline__ float sum_in_order(uint32_t e0, uint32_t e1, const Get& get) {
+    float sum = 0.0f;
+    for (uint32_t e = e0; e < e1; e += 4) {
+        float part[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) part[k] = e + k < e1 ? get(e + k) : 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (e + k < e1) sum += part[k];
+    }
+    return sum;
+}
+
 template <int ES, bool REORDER>
 __global__ __launch_bounds__(kReduceThreads)
 void nz_matvec_reduce_kernel(const uint32_t* __restrict__ row_index, const float* __restrict__ partials,
                              uint32_t batch, ReduceGroup g) {
     const uint32_t n = blockIdx.x * kReduceThreads + threadIdx.x;
     if (n >= g.total_rows) return;
-    uint32_t w = 0;
-#pragma unroll
-    for (uint32_t k = 1; k < NZ_MATVEC_MAX_WEIGHTS; ++k)
-        if (k < g.count && n >= g.row_base[k]) w = k;
-    const uint32_t local = n - g.row_base[w];
-    const uint8_t* bias = g.bias[w];
-    const float add = bias == nullptr ? 0.0f
-                      : word_to_float<ES, REORDER>(ES == 2 ? reinterpret_cast<const uint16_t*>(bias)[local]
-                                                           : reinterpret_cast<const uint32_t*>(bias)[local]);
+    const uint32_t w = weight_of(g, n), local = n - g.row_base[w];
+    const float add = row_bias<ES, REORDER>(g, w, local);
     const uint32_t e0 = row_index[n], e1 = row_index[n + 1];
     for (uint32_t b = 0; b < batch; ++b) {
-        // the row's partial sums are adjacent; four loads in flight at a
-        // time, the additions in position (element) order
-        float sum = 0.0f;
-        for (uint32_t e = e0; e < e1; e += 4) {
-            float part[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                part[k] = e + k < e1 ? partials[(e + k) * batch + b] : 0.0f;
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                if (e + k < e1) sum += part[k];
-        }
+        const float sum = sum_in_order(e0, e1, [&](uint32_t e) { return partials[e * batch + b]; });
+        store_result<ES, REORDER>(g.y[w], b * g.rows[w] + local, sum + add);
+    }
+}
+
+// LDS words a row segment has for its rows' first positions (rows + 1) and
+// partial sums (entries * BT): what two workgroups leave of a CU's 160 KB.
+template <int ES, int BT>
+constexpr uint32_t row_words() {
+    return static_cast<uint32_t>((160 * 1024 / 2 - sizeof(GroupLds<ES, matvec_waves<BT>()>)) / sizeof(uint32_t));
+}
+
+template <int ES, int BT>
+struct RowLds {
+    GroupLds<ES, matvec_waves<BT>()> group;   // first: its claim counter must sit in the first 64 KB
+    uint32_t words[row_words<ES, BT>()];
+};
+
+// The whole product in one launch, for plans whose workgroups own their rows
+// (nz_row_work): nz_matvec_kernel with the partial sums in LDS, added up in
+// the same order by the workgroup itself after its last tile. The two-launch
+// form needs a second kernel that mostly waits: 4 us of its own and 3 us
+// between the two on every product, whatever its size. 28672 x 4096 bf16
+// weights took 52.2 us in two launches and 45.2 in one, 6144 x 4096 for four
+// rows 22.3 and 21.4 (then bound by the host's calls).
+template <int ES, bool REORDER, bool LONG, int BT>
+__global__ __launch_bounds__(matvec_threads<BT>()) __attribute__((amdgpu_waves_per_eu(BT <= 2 ? 8 : 6)))
+void nz_matvec_rows_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __restrict__ frags,
+                           const nz_matvec_tile* __restrict__ tiles, const nz_row_work* __restrict__ segs,
+                           uint32_t cols, const uint8_t* __restrict__ xp, uint32_t batch,
+                           const uint32_t* __restrict__ row_index, ReduceGroup g) {
+    __shared__ __align__(16) RowLds<ES, BT> lds;
+    const uint32_t lane = lane_index();
+    const nz_row_work seg = segs[blockIdx.x];
+    const Activations<BT> x = activations<ES, BT>(xp, cols, batch);
+    // the host checks that starts and sums fit; the clamps keep a malformed
+    // segment's inside the array
+    constexpr uint32_t kWords = row_words<ES, BT>();
+    const uint32_t rows = min(seg.row1 - seg.row0, kWords - 1);
+    const uint32_t entries = min(seg.entries, (kWords - 1 - rows) / BT);
+    uint32_t* sums = lds.words + rows + 1;
+    for (uint32_t i = threadIdx.x; i <= rows; i += matvec_threads<BT>())
+        lds.words[i] = min(row_index[seg.row0 + i] - seg.entry0, entries);
+    if (threadIdx.x == 0) lds.group.claim[0] = 0;
+    if (seg.kind != NZ_KIND_RAW)
+        load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.group.lut, threadIdx.x);
+    __syncthreads();
+    run_segment<ES, REORDER, LONG, BT>(base, tiles + seg.tile0, seg.tile1 - seg.tile0, seg.kind, lds.group, lane, cols,
+                                       x, RowSums<BT>{sums, seg.entry0, entries});
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < rows * batch; i += matvec_threads<BT>()) {
+        const uint32_t b = i / rows, row = i - b * rows, n = seg.row0 + row;
+        const uint32_t w = weight_of(g, n), local = n - g.row_base[w];
+        const float add = row_bias<ES, REORDER>(g, w, local);
+        const float sum = sum_in_order(lds.words[row], lds.words[row + 1],
+                                       [&](uint32_t e) { return __uint_as_float(sums[e * BT + b]); });
         store_result<ES, REORDER>(g.y[w], b * g.rows[w] + local, sum + add);
     }
 }
@@ -510,6 +609,46 @@ hipError_t launch_batch(const void* base, const void* frags, const void* tiles, 
     if (batch <= 2) return NZ_MATVEC(2);
     return NZ_MATVEC(4);
 #undef NZ_MATVEC
+}
+
+template <int ES, bool REORDER, bool LONG, int BT>
+hipError_t launch_rows(const void* base, const void* frags, const void* tiles, const void* segs, uint32_t n_segs,
+                       uint32_t cols, const void* x, uint32_t batch, const uint32_t* row_index, const ReduceGroup& g,
+                       hipStream_t stream) {
+    hipLaunchKernelGGL((nz_matvec_rows_kernel<ES, REORDER, LONG, BT>), dim3(n_segs), dim3(matvec_threads<BT>()), 0,
+                       stream, static_cast<const uint8_t*>(base), static_cast<const nz_frag_desc*>(frags),
+                       static_cast<const nz_matvec_tile*>(tiles), static_cast<const nz_row_work*>(segs), cols,
+                       static_cast<const uint8_t*>(x), batch, row_index, g);
+    return hipGetLastError();
+}
+
+template <int ES, bool REORDER, bool LONG>
+hipError_t launch_rows_batch(const void* base, const void* frags, const void* tiles, const void* segs, uint32_t n_segs,
+                             uint32_t cols, const void* x, uint32_t batch, const uint32_t* row_index,
+                             const ReduceGroup& g, hipStream_t stream) {
+#define NZ_ROWS(BT) launch_rows<ES, REORDER, LONG, BT>(base, frags, tiles, segs, n_segs, cols, x, batch, row_index, g, stream)
+    if (batch <= 1) return NZ_ROWS(1);
+    if (batch <= 2) return NZ_ROWS(2);
+    return NZ_ROWS(4);
+#undef NZ_ROWS
+}
+
+template <int ES>
+uint32_t row_words_of(uint32_t batch) {
+    return batch <= 1 ? row_words<ES, 1>() : batch <= 2 ? row_words<ES, 2>() : row_words<ES, 4>();
+}
+
+ReduceGroup reduce_group(const nz_matvec_weight* weights, uint32_t n_weights) {
+    ReduceGroup g = {};
+    g.count = n_weights;
+    for (uint32_t k = 0; k < n_weights; ++k) {
+        g.y[k] = static_cast<uint8_t*>(weights[k].y);
+        g.bias[k] = static_cast<const uint8_t*>(weights[k].bias);
+        g.rows[k] = weights[k].rows;
+        g.row_base[k] = g.total_rows;
+        g.total_rows += weights[k].rows;
+    }
+    return g;
 }
 
 bool layout_ok(int element_size, int bit_reorder, char* message, size_t message_size) {
@@ -558,15 +697,7 @@ extern "C" int nz_hip_matvec_reduce(const uint32_t* row_index, const nz_matvec_w
                                     int bit_reorder, void* stream, char* message, size_t message_size) {
     if (n_weights == 0 || batch == 0) return 0;
     if (!layout_ok(element_size, bit_reorder, message, message_size)) return -1;
-    ReduceGroup g = {};
-    g.count = n_weights;
-    for (uint32_t k = 0; k < n_weights; ++k) {
-        g.y[k] = static_cast<uint8_t*>(weights[k].y);
-        g.bias[k] = static_cast<const uint8_t*>(weights[k].bias);
-        g.rows[k] = weights[k].rows;
-        g.row_base[k] = g.total_rows;
-        g.total_rows += weights[k].rows;
-    }
+    const ReduceGroup g = reduce_group(weights, n_weights);
     if (g.total_rows == 0) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid((g.total_rows + kReduceThreads - 1) / kReduceThreads);
@@ -582,6 +713,39 @@ extern "C" int nz_hip_matvec_reduce(const uint32_t* row_index, const nz_matvec_w
     const hipError_t rc = hipGetLastError();
     if (rc != hipSuccess) {
         snprintf(message, message_size, "matvec reduce launch failed: %s", hipGetErrorString(rc));
+        return -6;
+    }
+    return 0;
+}
+
+// LDS words a row segment has at `batch` activation rows, for its rows + 1
+// first positions and its entries (times 1, 2 or 4 sums).
+extern "C" uint32_t nz_hip_matvec_row_words(int element_size, uint32_t batch) {
+    return element_size == 2 ? row_words_of<2>(batch) : row_words_of<4>(batch);
+}
+
+// A product's row segments of one codebook kind: each output row of the
+// segments, complete.
+extern "C" int nz_hip_matvec_rows(const void* base, const void* frags, const void* tiles, const void* segs,
+                                  uint32_t n_segs, int element_size, int bit_reorder, int long_codes,
+                                  const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, const void* x,
+                                  uint32_t batch, const uint32_t* row_index, void* stream, char* message,
+                                  size_t message_size) {
+    if (n_segs == 0) return 0;
+    if (!layout_ok(element_size, bit_reorder, message, message_size)) return -1;
+    const ReduceGroup g = reduce_group(weights, n_weights);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t rc;
+#define NZ_BATCH(E, R, L) launch_rows_batch<E, R, L>(base, frags, tiles, segs, n_segs, cols, x, batch, row_index, g, st)
+    if (element_size == 2 && bit_reorder)
+        rc = long_codes ? NZ_BATCH(2, true, true) : NZ_BATCH(2, true, false);
+    else if (element_size == 2)
+        rc = long_codes ? NZ_BATCH(2, false, true) : NZ_BATCH(2, false, false);
+    else
+        rc = long_codes ? NZ_BATCH(4, true, true) : NZ_BATCH(4, true, false);
+#undef NZ_BATCH
+    if (rc != hipSuccess) {
+        snprintf(message, message_size, "matvec launch failed: %s", hipGetErrorString(rc));
         return -6;
     }
     return 0;

@@ -256,6 +256,9 @@ void pack_fragment(const Fragment& f, uint8_t* dst, uint64_t offset, uint64_t lu
 }
 
 constexpr uint64_t kMinTilesPerGroup = 16;
+// Elements that a row segment may have above its share: a workgroup takes
+// about 2.5 us for as many, less than the reduce launch it saves (7 us).
+constexpr double kMaxRowExcess = 16384;
 constexpr size_t kXcds = 8;   // MI355X: accelerator dies, each with its own L2
 
 void check_matvec_group(const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, unsigned element_size) {
@@ -391,6 +394,31 @@ void matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* ti
 
 namespace {
 
+// `groups` workgroups among runs of these costs: one each, the others by
+// largest remainder.
+std::vector<uint64_t> divide(const std::vector<double>& cost, uint64_t groups) {
+    const size_t n_seg = cost.size();
+    std::vector<uint64_t> share(n_seg, 1);
+    double total = 0;
+    for (double c : cost) total += c;
+    if (groups > n_seg && total > 0) {
+        // largest remainder over the workgroups left after one per segment
+        const uint64_t extra = groups - n_seg;
+        std::vector<std::pair<double, size_t>> rest;
+        uint64_t given = 0;
+        for (size_t i = 0; i < n_seg; ++i) {
+            const double exact = extra * cost[i] / total;
+            const uint64_t whole = static_cast<uint64_t>(exact);
+            share[i] += whole;
+            given += whole;
+            rest.push_back({exact - whole, i});
+        }
+        std::sort(rest.begin(), rest.end(), [](auto& x, auto& y) { return x.first > y.first || (x.first == y.first && x.second < y.second); });
+        for (size_t k = 0; given < extra; ++k, ++given) share[rest[k % n_seg].second] += 1;
+    }
+    return share;
+}
+
 // Maximal runs of one LUT and kind, their costs (elements, raw tiles at half
 // weight) and the workgroups each run gets.
 struct Shares {
@@ -427,25 +455,7 @@ Shares share_out(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_til
     // so it should have at least a tile per wavefront to decode.
     const uint64_t enough = (n_tiles + kMinTilesPerGroup - 1) / kMinTilesPerGroup;
     const uint64_t groups = std::max<uint64_t>(std::min<uint64_t>(slots, enough), n_seg);
-    std::vector<uint64_t>& share = out.share;
-    share.assign(n_seg, 1);
-    double total = 0;
-    for (double c : cost) total += c;
-    if (groups > n_seg && total > 0) {
-        // largest remainder over the workgroups left after one per segment
-        const uint64_t extra = groups - n_seg;
-        std::vector<std::pair<double, size_t>> rest;
-        uint64_t given = 0;
-        for (size_t i = 0; i < n_seg; ++i) {
-            const double exact = extra * cost[i] / total;
-            const uint64_t whole = static_cast<uint64_t>(exact);
-            share[i] += whole;
-            given += whole;
-            rest.push_back({exact - whole, i});
-        }
-        std::sort(rest.begin(), rest.end(), [](auto& x, auto& y) { return x.first > y.first || (x.first == y.first && x.second < y.second); });
-        for (size_t k = 0; given < extra; ++k, ++given) share[rest[k % n_seg].second] += 1;
-    }
+    out.share = divide(cost, groups);
     return out;
 }
 
@@ -498,6 +508,71 @@ std::vector<nz_work> plan_work(const nz_frag_desc* frags, const nz_tile* tiles, 
         }
     }
     return ranges;
+}
+
+std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
+                                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
+                                   unsigned element_size, uint32_t slots, double first_weight) {
+    if (!(first_weight >= 1.0 && first_weight <= 16.0)) fail(kInvalidArgument, "first_weight must be in [1, 16].");
+    std::vector<uint32_t> row_index, entries;
+    plan_matvec(frags, tiles, n_tiles, weights, n_weights, cols, element_size, row_index, entries);
+    const uint32_t n_rows = static_cast<uint32_t>(row_index.size()) - 1;
+    auto key = [&](uint32_t t) {
+        const nz_frag_desc& f = frags[tiles[t].frag];
+        return std::pair<uint64_t, uint32_t>(f.kind == NZ_KIND_RAW ? 0 : f.lut, f.kind);
+    };
+    // entries[e] / 2 is the tile of partial position e: row n's tiles are
+    // those of positions row_index[n] .. row_index[n + 1]
+    auto first = [&](uint32_t n) { return entries[row_index[n]] / 2; };
+    auto last = [&](uint32_t n) { return entries[row_index[n + 1] - 1] / 2; };
+    std::vector<nz_row_work> runs;   // maximal runs of rows whose tiles follow each other with one LUT and kind
+    std::vector<double> cost;
+    for (uint32_t n = 0; n < n_rows; ++n) {
+        for (uint32_t e = row_index[n] + 1; e < row_index[n + 1]; ++e)
+            if (entries[e] / 2 != entries[e - 1] / 2 + 1 || key(entries[e] / 2) != key(first(n))) return {};
+        const bool joins = n && key(first(n)) == key(last(n - 1)) && first(n) - last(n - 1) <= 1u;
+        if (!joins) {
+            runs.push_back({0, 0, 0, key(first(n)).second, n, n, 0, 0});
+            cost.push_back(0);
+        }
+        runs.back().row1 = n + 1;
+        cost.back() += runs.back().kind == NZ_KIND_RAW ? 0.5 * cols : cols;   // as share_out counts them
+    }
+    const uint64_t enough = (n_tiles + kMinTilesPerGroup - 1) / kMinTilesPerGroup;
+    std::vector<uint64_t> share = divide(cost, std::max<uint64_t>(std::min<uint64_t>(slots, enough), runs.size()));
+    uint64_t total = 0;
+    bool any_long = false, any_other = false;
+    for (size_t i = 0; i < runs.size(); ++i) {
+        share[i] = std::min<uint64_t>(share[i], runs[i].row1 - runs[i].row0);
+        total += share[i];
+        (runs[i].kind == NZ_KIND_LONG ? any_long : any_other) = true;
+    }
+    // the weights of plan_work
+    const bool paired = first_weight != 1.0 && total == slots && slots % 2 == 0 && !(any_long && any_other);
+    auto weight = [&](uint64_t b) { return paired && b < slots / 2 ? first_weight : 1.0; };
+    std::vector<nz_row_work> out;
+    for (size_t i = 0; i < runs.size(); ++i) {
+        const nz_row_work& run = runs[i];
+        const uint64_t parts = share[i], base = out.size();
+        const uint32_t rows = run.row1 - run.row0;
+        double weights_sum = 0, reached = 0;
+        for (uint64_t j = 0; j < parts; ++j) weights_sum += weight(base + j);
+        uint32_t row = run.row0;
+        for (uint64_t j = 0; j < parts; ++j) {
+            reached += weight(base + j);
+            // the nearest row to the share's end that leaves every segment a row
+            const uint32_t want = run.row0 + static_cast<uint32_t>(rows * (reached / weights_sum) + 0.5);
+            const uint32_t end = j + 1 == parts ? run.row1
+                                 : std::min<uint32_t>(std::max(want, row + 1),
+                                                      run.row1 - static_cast<uint32_t>(parts - j - 1));
+            const double excess = (end - row) - rows * weight(base + j) / weights_sum;   // rows above the exact share
+            if (excess * cols > kMaxRowExcess && excess > 0.1 * (end - row)) return {};
+            out.push_back({first(row), last(end - 1) + 1, tiles[first(row)].frag, run.kind, row, end, row_index[row],
+                           row_index[end] - row_index[row]});
+            row = end;
+        }
+    }
+    return out;
 }
 
 std::vector<nz_work> plan_work_interleaved(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,

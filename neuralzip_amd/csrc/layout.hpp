@@ -95,6 +95,16 @@ void matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* ti
                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, unsigned element_size,
                   uint64_t store_bytes, nz_matvec_tile* out);
 
+// Row segments of the same product: one per workgroup, each owning whole
+// rows of the stacked output, with the shares of plan_work cut at rows.
+// Empty where some row's tiles are not adjacent in the launch order with one
+// LUT and kind, or where cutting at rows would load a segment with over
+// kMaxRowExcess elements and a tenth more than its share. Fails where
+// plan_matvec would.
+std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
+                                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
+                                   unsigned element_size, uint32_t slots, double first_weight);
+
 // CPU emulation of the decode kernel over a packed buffer; writes words
 // into `out` (the output workspace image).
 void emulate_decode(const uint8_t* base, const nz_frag_desc* frags, const nz_tile* tiles,

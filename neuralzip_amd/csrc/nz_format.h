@@ -141,6 +141,19 @@ struct nz_matvec_tile {          // 40 bytes
     uint32_t col0;               // column of the first vector's first element
 };
 
+// A *row segment*: the work of one workgroup that owns output rows of a fused
+// product, so that it can add up its rows' partial sums itself. Its tiles
+// cover rows [row0, row1) of the stacked output; where a tile at either end
+// also touches a neighbour's row, both segments decode it and each keeps its
+// own rows' sums: partial positions [entry0, entry0 + entries).
+struct nz_row_work {             // 32 bytes
+    uint32_t tile0, tile1;
+    uint32_t lut_frag;
+    uint32_t kind;
+    uint32_t row0, row1;
+    uint32_t entry0, entries;
+};
+
 // Raw lanes and raw exponent lanes are stored with `out % V` leading pad
 // bytes (V elements per 16-byte vector) so that a vector-aligned output
 // element maps to a vector-aligned lane address.

@@ -202,6 +202,16 @@ class HIPDecoder:
                 t = torch.from_numpy(group.view(np.uint8).copy()).to(device)
                 tensors.append(t)
                 launches.append((t.data_ptr(), len(group), long_codes))
+        # the same product in one launch, where workgroups can own whole rows
+        row_segments, words = _native.matvec_row_plan(store.descs, tiles, weights, cols, dtype.element_size, slots,
+                                                      first_weight)
+        is_long = row_segments["kind"] == KIND_LONG
+        row_groups = []
+        for long_codes, group in enumerate((row_segments[~is_long], row_segments[is_long])):
+            if len(group):
+                t = torch.from_numpy(group.view(np.uint8).copy()).to(device)
+                tensors.append(t)
+                row_groups.append((t.data_ptr(), len(group), long_codes))
         descs = store.descs[fragment_indices]
         numel = descs["numel"].astype(np.int64)
         raw = descs["kind"] == KIND_RAW
@@ -214,8 +224,18 @@ class HIPDecoder:
                              n_segments, es, reorder, long_codes, int(cols))
                             for segments_ptr, n_segments, long_codes in launches)
         reduce_args = (tensors[1].data_ptr(), ctypes.addressof(reduce_weights), len(weights))
+        # per activation row count: the one-launch form's fixed arguments, or
+        # None where its partial sums do not fit a workgroup's LDS
+        row_args = []
+        for batch in range(1, _native.MATVEC_MAX_BATCH + 1):
+            need = words[min(batch - 1, 2)]
+            fits = row_groups and need <= _native.lib().nz_matvec_row_words(es, batch)
+            row_args.append(tuple((store.buffer.data_ptr(), store.frags.data_ptr(), tensors[0].data_ptr(), segments_ptr,
+                                   n_segments, need, es, reorder, long_codes, ctypes.addressof(reduce_weights),
+                                   len(weights), int(cols))
+                                  for segments_ptr, n_segments, long_codes in row_groups) if fits else None)
         return PreparedMatvec(tuple(tensors), device, key[:2], dtype.torch_dtype, weights, int(cols), len(tiles),
-                              store, tuple(launches), reads, reduce_weights, launch_args, reduce_args)
+                              store, tuple(launches), reads, reduce_weights, launch_args, reduce_args, tuple(row_args))
 
     def matvec(self, prepared, x, biases=None, partials=None, stream=None):
         """x @ W^T (+ bias) for each weight of the product: x is (batch, cols),
@@ -249,7 +269,8 @@ class HIPDecoder:
         # them to that stream.
         with torch.cuda.stream(stream):
             x = x.contiguous()
-            if partials is None:
+            row_args = prepared.row_args[batch - 1]
+            if partials is None and row_args is None:
                 partials = torch.empty(need, dtype=torch.float32, device=prepared.device)
             # one allocation; weight k's (batch, rows) output is a contiguous block of it
             out = torch.empty(batch * prepared.total_rows, dtype=prepared.dtype, device=prepared.device)
@@ -260,7 +281,14 @@ class HIPDecoder:
             reduce_weights[k].y = block.data_ptr()
             reduce_weights[k].bias = None if bias is None else bias.data_ptr()
         lib, es, reorder = _native.lib(), prepared.layout[0], int(prepared.layout[1])
-        x_ptr, partials_ptr, stream_ptr = x.data_ptr(), partials.data_ptr(), stream.cuda_stream
+        x_ptr, stream_ptr = x.data_ptr(), stream.cuda_stream
+        if row_args is not None:   # workgroups that own their rows: one launch, no partial sums in memory
+            for args in row_args:
+                rc = lib.nz_matvec_rows(*args, x_ptr, batch, prepared.reduce_args[0], stream_ptr)
+                if rc:
+                    _native.check(rc)
+            return tuple(ys)
+        partials_ptr = partials.data_ptr()
         for args in prepared.launch_args:
             rc = lib.nz_matvec_launch(*args, x_ptr, batch, partials_ptr, prepared.n_tiles, stream_ptr)
             if rc:
@@ -303,6 +331,9 @@ class PreparedMatvec:
     # the launches' and the reduce's fixed leading arguments, built once
     launch_args: tuple = field(repr=False, default=())
     reduce_args: tuple = field(repr=False, default=())
+    # for 1 .. MATVEC_MAX_BATCH activation rows: the one-launch form's
+    # arguments per launch, or None where the two passes run instead
+    row_args: tuple = field(repr=False, default=(None,) * _native.MATVEC_MAX_BATCH)
 
     @property
     def rows(self):
