@@ -150,18 +150,26 @@ __device__ void raw_tile(const uint8_t* __restrict__ base, const nz_frag_desc& f
 }
 
 
-// One wavefront's share of a Huffman segment: claim tiles until the segment
+// Whether a wavefront's first tile is requested before the LUT copy ends (the
+// kernel for 32-bit words has no registers left to hold it).
+constexpr bool first_early(int es) { return es == 2; }
+
+// One wavefront's share of a Huffman segment: tile `t` < n (with first_early
+// described by `cur`, its bits requested into `fc`), then claimed tiles until the segment
 // is used up, fetching (and claiming) one tile ahead of the one it decodes.
 template <int ES, bool REORDER, bool LONG, bool ESC, bool CACHED>
 __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_frag_desc* frags, const nz_tile* tiles,
                                                 const nz_work& seg, uint32_t* counter, uint32_t lane,
-                                                const uint32_t* lut, uint8_t* stage, uint8_t* out) {
+                                                const uint32_t* lut, uint8_t* stage, uint8_t* out, uint32_t t,
+                                                TileInfo cur, Fetch<ES, LONG> fc) {
     const uint32_t n = seg.tile1 - seg.tile0;
-    uint32_t t = claim(counter);
-    if (t >= n) return;
-    TileInfo cur = tile_info<ES>(base, frags, tiles, seg.tile0 + t);
-    Fetch<ES, LONG> fc;
-    fetch_bits<ES, LONG>(cur, lane, fc);
+    if (!first_early(ES)) {
+        t = claim(counter);
+        if (t >= n) return;
+        cur = tile_info<ES>(base, frags, tiles, seg.tile0 + t);
+        fetch_bits<ES, LONG>(cur, lane, fc);
+    }
+    asm volatile("");   // keeps what the kernel's two instances of this share from moving ahead of both, to spill there
     // Raw lanes are requested a tile ahead, but for long codes of 32-bit
     // words, where the next tile's twelve registers would spill.
     constexpr bool kAhead = !(ES == 4 && LONG);
@@ -211,26 +219,40 @@ void nz_decode_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __re
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NZ_WAVE);
     const uint32_t lane = lane_index();
     const nz_work seg = segs[blockIdx.x];
-    if (threadIdx.x == 0) lds.claim[0] = 0;
     if (seg.kind == NZ_KIND_RAW) {
+        if (threadIdx.x == 0) lds.claim[0] = 0;
         __syncthreads();
         raw_segment<ES, REORDER>(base, frags, tiles, seg, lds.claim, lane, out);
         return;
     }
-    load_lut<REORDER, WAVES * NZ_WAVE>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
+    // With first_early, a wavefront's first tile is the one of its index and
+    // claims start behind those. Its bits are requested beside the LUT, so
+    // that a workgroup with few tiles waits for both at once.
+    const uint32_t n = seg.tile1 - seg.tile0;
+    if (threadIdx.x == 0) lds.claim[0] = first_early(ES) ? WAVES * NZ_WAVE : 0;
+    LutCopy<REORDER, WAVES * NZ_WAVE> lut;
+    lut.fetch(base + frags[seg.lut_frag].lut, threadIdx.x);
+    TileInfo first;
+    Fetch<ES, LONG> data;
+    if (first_early(ES)) {
+        first = tile_info<ES>(base, frags, tiles, seg.tile0 + min(wave, n - 1));
+        fetch_bits<ES, LONG>(first, lane, data);
+    }
+    lut.store(lds.lut, threadIdx.x);
     __syncthreads();
+    if (first_early(ES) && wave >= n) return;
     // Codebooks whose codes all fit the primary table run the loop without
     // the escape check (long-code codebooks always have escapes).
     if constexpr (LONG) {
         huffman_segment<ES, REORDER, true, true, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut, lds.stage[wave],
-                                                         out);
+                                                         out, wave, first, data);
     } else {
         if (lds.lut[0])
             huffman_segment<ES, REORDER, false, true, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut,
-                                                              lds.stage[wave], out);
+                                                              lds.stage[wave], out, wave, first, data);
         else
             huffman_segment<ES, REORDER, false, false, CACHED>(base, frags, tiles, seg, lds.claim, lane, lds.lut,
-                                                               lds.stage[wave], out);
+                                                               lds.stage[wave], out, wave, first, data);
     }
 }
 

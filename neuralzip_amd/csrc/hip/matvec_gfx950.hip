@@ -451,8 +451,11 @@ void nz_matvec_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __re
     const nz_work seg = segs[blockIdx.x];
     const Activations<BT> x = activations<ES, BT>(xp, cols, batch);
     if (threadIdx.x == 0) lds.claim[0] = 0;
-    if (seg.kind != NZ_KIND_RAW)
-        load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.lut, threadIdx.x);
+    if (seg.kind != NZ_KIND_RAW) {
+        LutCopy<REORDER, matvec_threads<BT>()> lut;
+        lut.fetch(base + frags[seg.lut_frag].lut, threadIdx.x);
+        lut.store(lds.lut, threadIdx.x);
+    }
     __syncthreads();
     run_segment<ES, REORDER, LONG, BT>(base, tiles + seg.tile0, seg.tile1 - seg.tile0, seg.kind, lds, lane, cols, x,
                                        GlobalSums{partials, batch});
@@ -570,11 +573,14 @@ void nz_matvec_rows_kernel(const uint8_t* __restrict__ base, const nz_frag_desc*
     const uint32_t rows = min(seg.row1 - seg.row0, kWords - 1);
     const uint32_t entries = min(seg.entries, (kWords - 1 - rows) / BT);
     uint32_t* sums = lds.words + rows + 1;
+    if (threadIdx.x == 0) lds.group.claim[0] = 0;
+    if (seg.kind != NZ_KIND_RAW) {
+        LutCopy<REORDER, matvec_threads<BT>()> lut;
+        lut.fetch(base + frags[seg.lut_frag].lut, threadIdx.x);
+        lut.store(lds.group.lut, threadIdx.x);
+    }
     for (uint32_t i = threadIdx.x; i <= rows; i += matvec_threads<BT>())
         lds.words[i] = min(row_index[seg.row0 + i] - seg.entry0, entries);
-    if (threadIdx.x == 0) lds.group.claim[0] = 0;
-    if (seg.kind != NZ_KIND_RAW)
-        load_lut<REORDER, matvec_threads<BT>()>(base + frags[seg.lut_frag].lut, lds.group.lut, threadIdx.x);
     __syncthreads();
     run_segment<ES, REORDER, LONG, BT>(base, tiles + seg.tile0, seg.tile1 - seg.tile0, seg.kind, lds.group, lane, cols,
                                        x, RowSums<BT>{sums, seg.entry0, entries});

@@ -418,29 +418,61 @@ __device__ __forceinline__ void decode_tile(LaneDecode l, const uint32_t* lut) {
     wave_lds_sync();
 }
 
-// Copies a segment's LUT image into LDS, its bytes in staged form.
+// A segment's LUT image on its way into LDS: the header and the primary
+// entries, whose place and number are the same in every image, are requested
+// at once by fetch(); store() writes them in staged form and copies the
+// escape records and tokens behind them, whose number the header gives.
+// (Reading the size first, then copying in a loop that waits for each of its
+// loads, put four memory latencies one after the other ahead of a
+// workgroup's first tile; two are left. With the decode kernel's first tiles
+// requested beside it, 14.9 M bf16 elements went from 11.9 to 10.3 us and
+// 13.1 M fp32 elements from 18.2 to 17.5.)
 template <bool REORDER, int THREADS>
-__device__ __forceinline__ void load_lut(const uint8_t* image, uint32_t* lut, uint32_t thread) {
-    const uint4* img = reinterpret_cast<const uint4*>(image);
-    // the host checks every image against NZ_LUT_MAX_WORDS; the clamp keeps a
-    // malformed one from overwriting the staging areas behind the LUT
-    const uint32_t words = min(reinterpret_cast<const uint32_t*>(img)[2], uint32_t(NZ_LUT_MAX_WORDS));
-    const uint32_t tokens = NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * reinterpret_cast<const uint32_t*>(img)[0];
-    uint4* dst = reinterpret_cast<uint4*>(lut);
-    for (uint32_t i = thread; i < (words + 3) / 4; i += THREADS) {
-        uint4 v = img[i];
-        if (i >= 1 && i < 1 + NZ_LUT_ENTRIES / 2) {   // two primary entries
-            if (v.x >> NZ_ENTRY_COUNT) v.y = staged_form<REORDER>(v.y);
-            if (v.z >> NZ_ENTRY_COUNT) v.w = staged_form<REORDER>(v.w);
-        } else if (REORDER) {   // escape tokens: two bytes below the count
-            uint32_t* w = &v.x;
+struct LutCopy {
+    static constexpr uint32_t kPrimary = NZ_LUT_ENTRIES / 2;   // 16-byte vectors of two entries
+    static constexpr uint32_t kRounds = (kPrimary + THREADS - 1) / THREADS;
+    const uint4* image;
+    uint4 head;
+    uint4 v[kRounds];
+
+    __device__ __forceinline__ void fetch(const uint8_t* at, uint32_t thread) {
+        image = reinterpret_cast<const uint4*>(at);
+        head = image[0];
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                if (4 * i + k >= tokens) w[k] = bfi(0xFFFFu, staged_form<true>(w[k] & 0xFFFFu), w[k]);
-        }
-        dst[i] = v;
+        for (uint32_t r = 0; r < kRounds; ++r)
+            v[r] = image[1 + (kPrimary % THREADS ? min(thread + r * THREADS, kPrimary - 1) : thread + r * THREADS)];
     }
-}
+
+    __device__ __forceinline__ void store(uint32_t* lut, uint32_t thread) {
+        uint4* dst = reinterpret_cast<uint4*>(lut);
+        // the host checks every image against NZ_LUT_MAX_WORDS; the clamp keeps a
+        // malformed one from overwriting the staging areas behind the LUT
+        const uint32_t words = min(head.z, uint32_t(NZ_LUT_MAX_WORDS));
+        const uint32_t tokens = NZ_LUT_HEADER + 2 * NZ_LUT_ENTRIES + NZ_ESC_RECORD * head.x;
+        const uint32_t i = 1 + kPrimary + thread;   // escape records and tokens: 212 vectors at most
+        static_assert((NZ_LUT_MAX_WORDS + 3) / 4 - 1 - kPrimary <= THREADS, "one vector per thread");
+        const bool tail = i < (words + 3) / 4;
+        uint4 e = make_uint4(0u, 0u, 0u, 0u);
+        if (tail) e = image[i];
+        if (thread == 0) dst[0] = head;
+#pragma unroll
+        for (uint32_t r = 0; r < kRounds; ++r) {
+            if (kPrimary % THREADS != 0 && thread + r * THREADS >= kPrimary) break;
+            if (v[r].x >> NZ_ENTRY_COUNT) v[r].y = staged_form<REORDER>(v[r].y);
+            if (v[r].z >> NZ_ENTRY_COUNT) v[r].w = staged_form<REORDER>(v[r].w);
+            dst[1 + thread + r * THREADS] = v[r];
+        }
+        if (tail) {
+            if (REORDER) {   // escape tokens: two bytes below the count
+                uint32_t* w = &e.x;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+                    if (4 * i + k >= tokens) w[k] = bfi(0xFFFFu, staged_form<true>(w[k] & 0xFFFFu), w[k]);
+            }
+            dst[i] = e;
+        }
+    }
+};
 
 // A workgroup's LDS. The claim counter comes first: ds_append takes its
 // address from M0's low 16 bits, which reach the first 64 KB.
