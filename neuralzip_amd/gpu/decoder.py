@@ -6,6 +6,7 @@ device tensors per chunk (neuralzip/gpu/inference.py:401-432), every
 fragment of an export lives in one packed device buffer (DeviceStore); a
 PreparedBatch holds the tile and workgroup arrays of one launch.
 """
+import contextlib
 import ctypes
 from dataclasses import dataclass, field
 from functools import cached_property
@@ -27,10 +28,19 @@ SLOTS = None
 # time of the second (Llama-3-8B shapes), and the second then ran alone.
 # 1.75 evened them out best of 1.5, 1.75, 2 and 2.5.
 MATVEC_FIRST_WEIGHT = 1.75
+_CURRENT = contextlib.nullcontext()   # the calling thread's current stream
 
 
 def _align(value, alignment=256):
     return (value + alignment - 1) // alignment * alignment
+
+
+def _stream_handle(device, stream):
+    """The HIP stream of `stream`, or of the device's current one (None), as
+    an integer handle."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 class DeviceStore:
@@ -103,7 +113,7 @@ class PreparedBatch:
     output: torch.Tensor = field(repr=False)
     outputs: tuple = field(repr=False, default=())
     algorithmic_bytes: int = 0
-    # nz_decode_launch arguments but the stream, fixed at prepare time
+    # nz_decode_launch_ex arguments but the stream, fixed at prepare time
     launch_args: tuple = field(repr=False, default=())
 
 
@@ -262,32 +272,33 @@ class HIPDecoder:
         if partials is not None and (partials.dtype != torch.float32 or partials.numel() < need
                                      or partials.device != prepared.device):
             raise ValueError("matvec partials buffer is too small.")
-        if stream is None:
-            stream = torch.cuda.current_stream(prepared.device)
+        row_args = prepared.row_args[batch - 1]
         # The input copy and this call's own buffers are made on `stream`, so
         # they are ordered before the launches and the caching allocator ties
-        # them to that stream.
-        with torch.cuda.stream(stream):
+        # them to that stream. (Entering the current stream's context would
+        # cost a product as much host time as its launch.)
+        with torch.cuda.stream(stream) if stream is not None else _CURRENT:
             x = x.contiguous()
-            row_args = prepared.row_args[batch - 1]
             if partials is None and row_args is None:
                 partials = torch.empty(need, dtype=torch.float32, device=prepared.device)
             # one allocation; weight k's (batch, rows) output is a contiguous block of it
             out = torch.empty(batch * prepared.total_rows, dtype=prepared.dtype, device=prepared.device)
-        blocks = out.split([batch * rows for _, rows in prepared.weights])
-        reduce_weights, ys = prepared.reduce_weights, []
-        for k, ((_, rows), bias, block) in enumerate(zip(prepared.weights, biases, blocks)):
-            ys.append(block.view(batch, rows))
-            reduce_weights[k].y = block.data_ptr()
-            reduce_weights[k].bias = None if bias is None else bias.data_ptr()
-        lib, es, reorder = _native.lib(), prepared.layout[0], int(prepared.layout[1])
-        x_ptr, stream_ptr = x.data_ptr(), stream.cuda_stream
+        stream_ptr = _stream_handle(prepared.device, stream)
+        es, reorder, y_ptr = prepared.layout[0], int(prepared.layout[1]), out.data_ptr()
+        reduce_weights = prepared.reduce_weights
+        for item, (_, rows), bias in zip(reduce_weights, prepared.weights, biases):
+            item.y, item.bias = y_ptr, None if bias is None else bias.data_ptr()
+            y_ptr += batch * rows * es
+        sizes = [batch * rows for _, rows in prepared.weights]
+        ys = tuple(block.view(batch, rows) for block, (_, rows) in
+                   zip(out.split(sizes) if len(sizes) > 1 else (out,), prepared.weights))
+        lib, x_ptr = _native.lib(), x.data_ptr()
         if row_args is not None:   # workgroups that own their rows: one launch, no partial sums in memory
             for args in row_args:
                 rc = lib.nz_matvec_rows(*args, x_ptr, batch, prepared.reduce_args[0], stream_ptr)
                 if rc:
                     _native.check(rc)
-            return tuple(ys)
+            return ys
         partials_ptr = partials.data_ptr()
         for args in prepared.launch_args:
             rc = lib.nz_matvec_launch(*args, x_ptr, batch, partials_ptr, prepared.n_tiles, stream_ptr)
@@ -296,15 +307,14 @@ class HIPDecoder:
         rc = lib.nz_matvec_reduce(*prepared.reduce_args, partials_ptr, batch, es, reorder, stream_ptr)
         if rc:
             _native.check(rc)
-        return tuple(ys)
+        return ys
 
     def decode_batch(self, prepared, stream=None):
         """Launches the batch on `stream` (default: the current stream); the
         batch holds its device arrays, so the saved pointers stay valid."""
-        if stream is None:
-            stream = torch.cuda.current_stream(prepared.device)
-        *args, flags = prepared.launch_args
-        _native.decode_launch(*args, stream.cuda_stream, flags)
+        rc = _native.lib().nz_decode_launch_ex(*prepared.launch_args, _stream_handle(prepared.device, stream))
+        if rc:
+            _native.check(rc)
         return prepared.outputs
 
 
