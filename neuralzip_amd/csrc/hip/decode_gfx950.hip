@@ -103,7 +103,7 @@ __device__ __forceinline__ void store_tile(const TileInfo& ti, const Fetch<ES, L
         const bool partial = !(vec0 >= ti.s0 && vec0 + V <= ti.s1);
         const bool mine = lane < 2 * V && (lane < V || ti.nv > 1) && partial && g >= ti.s0 && g < ti.s1;
         store_element<ES, REORDER>(out, mine ? g * ES : kOutOfRange, stage[NZ_STAGE_ORIGIN + (mine ? g : 0u)],
-                                   d.edge);
+                                   edge_raw<ES>(ti, mine ? g : kOutOfRange));
     }
     wave_lds_sync();
 }

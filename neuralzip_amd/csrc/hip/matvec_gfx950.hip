@@ -298,8 +298,8 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
         const bool partial = !(vec0 >= ti.s0 && vec0 + V <= ti.s1);
         const bool mine = lane < 2 * V && (lane < V || ti.nv > 1) && partial && g >= ti.s0 && g < ti.s1;
         const uint32_t expo = stage[NZ_STAGE_ORIGIN + (mine ? g : 0u)];
-        const float wf = mine ? word_to_float<ES, REORDER>(element_word<ES, REORDER>(expo, d.edge))
-                              : 0.0f;
+        const uint32_t raw = edge_raw<ES>(ti, mine ? g : kOutOfRange);
+        const float wf = mine ? word_to_float<ES, REORDER>(element_word<ES, REORDER>(expo, raw)) : 0.0f;
         const bool h = g >= rs.split;
         const uint32_t off = mine ? (rs.col0 + g - (h ? cols : 0u)) * ES : kOutOfRange;
 #pragma unroll

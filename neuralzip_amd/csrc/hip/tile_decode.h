@@ -221,7 +221,6 @@ struct Fetch {
     uint32_t meta;
     uint32_t w[LONG ? 4 : 3];
     uint32_t raw[Geometry<ES>::kRounds][Geometry<ES>::kLaneWords];
-    uint32_t edge;             // raw lane bytes of this lane's edge element
 };
 
 // The part of a tile's data the decode needs first: window metadata and bits.
@@ -239,7 +238,7 @@ __device__ __forceinline__ void fetch_bits(const TileInfo& ti, uint32_t lane, Fe
     }
 }
 
-// The part used only after the decode: raw lanes and the edge elements' bytes.
+// The part used only after the decode: raw lanes.
 template <int ES, bool LONG>
 __device__ __forceinline__ void fetch_raw(const TileInfo& ti, uint32_t lane, Fetch<ES, LONG>& d) {
     using G = Geometry<ES>;
@@ -258,14 +257,21 @@ __device__ __forceinline__ void fetch_raw(const TileInfo& ti, uint32_t lane, Fet
             d.raw[r][2] = __builtin_amdgcn_raw_buffer_load_b32(lanes, at + 2 * ti.stride, 0, 0);
         }
     }
-    const uint32_t g = lane < 2 * G::V ? edge_index<ES>(ti, lane) : kOutOfRange;
-    if (ES == 2) {
-        d.edge = __builtin_amdgcn_raw_buffer_load_b8(lanes, g, 0, 0);
-    } else {
-        d.edge = __builtin_amdgcn_raw_buffer_load_b8(lanes, g, 0, 0) |
-                 (static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(lanes, g + ti.stride, 0, 0)) << 8) |
-                 (static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(lanes, g + 2 * ti.stride, 0, 0)) << 16);
-    }
+}
+
+// Raw lane bytes (lane k in byte k) of the element at staging index g of one
+// of a tile's partial vectors, 0 for a lane without one (kOutOfRange). Tiles
+// end on whole vectors but at a fragment's unaligned ends, so the load is
+// left to the tiles that have such elements.
+template <int ES>
+__device__ __forceinline__ uint32_t edge_raw(const TileInfo& ti, uint32_t g) {
+    const uint32_t span = ti.nv * Geometry<ES>::V;
+    const rsrc_t lanes = make_rsrc(ti.lanes, ES == 2 ? span : 2 * ti.stride + span);
+    uint32_t raw = __builtin_amdgcn_raw_buffer_load_b8(lanes, g, 0, 0);
+    if (ES == 4)
+        raw |= (static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(lanes, g + ti.stride, 0, 0)) << 8) |
+               (static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(lanes, g + 2 * ti.stride, 0, 0)) << 16);
+    return raw;
 }
 
 __device__ __forceinline__ uint2 lut_entry(const uint32_t* lut, uint32_t w0) {
