@@ -314,8 +314,9 @@ int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights,
 /* Plan of the same product for one launch without partial sums in device
  * memory: segments (one workgroup each, 32 bytes, caller-allocated for
  * `capacity`) whose workgroups own whole rows and add up their rows
- * themselves. Tiles, weights, slots and first_weight as for nz_matvec_plan
- * and nz_plan_work. *n_segments receives 0 where the product has no such
+ * themselves. Tiles, row_index (host, n_rows + 1 values) and entries as
+ * nz_matvec_plan took and gave them, slots and first_weight as for
+ * nz_plan_work. *n_segments receives 0 where the product has no such
  * plan: a row in tiles of two codebooks or of separate places of the launch
  * order, or rows so long that whole rows would leave the workgroups
  * unevenly loaded. words[i] (i = 0, 1, 2) receives the LDS words that the
@@ -323,8 +324,8 @@ int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights,
  * takes at most nz_matvec_row_words. No counterpart in the reference (see
  * nz_matvec_plan). */
 int nz_matvec_row_plan(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
-                       const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, int element_size,
-                       uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
+                       const uint32_t* row_index, uint32_t n_rows, const uint32_t* entries, uint32_t n_entries,
+                       uint32_t cols, uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
                        uint32_t* n_segments, uint32_t* words);
 
 /* LDS words one row segment may need at `batch` activation rows. */

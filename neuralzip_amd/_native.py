@@ -129,7 +129,7 @@ def lib():
         L.nz_matvec_launch.argtypes = [vp, vp, vp, vp, u32, ctypes.c_int, ctypes.c_int, ctypes.c_int, u32, vp, u32,
                                        vp, u32, vp]
         L.nz_matvec_reduce.argtypes = [vp, vp, u32, vp, u32, ctypes.c_int, ctypes.c_int, vp]
-        L.nz_matvec_row_plan.argtypes = [vp, vp, u32, vp, u32, u32, ctypes.c_int, u32, ctypes.c_double, vp, u32,
+        L.nz_matvec_row_plan.argtypes = [vp, vp, u32, vp, u32, vp, u32, u32, u32, ctypes.c_double, vp, u32,
                                          ctypes.POINTER(u32), vp]
         L.nz_matvec_row_words.argtypes = [ctypes.c_int, u32]
         L.nz_matvec_row_words.restype = u32
@@ -383,15 +383,15 @@ def matvec_tiles(descs, tiles, weights, cols, element_size, store_bytes):
     return out
 
 
-def matvec_row_plan(descs, tiles, weights, cols, element_size, slots, first_weight=1.0):
+def matvec_row_plan(descs, tiles, row_index, entries, cols, slots, first_weight=1.0):
     """Row segments (ROW_WORK; empty where the product has none) and the LDS
-    words the largest one needs for up to 1, 2 and 4 activation rows."""
-    array = matvec_weights(weights)
-    rows = sum(int(w[1]) for w in weights)
+    words the largest one needs for up to 1, 2 and 4 activation rows, from
+    matvec_plan's row_index and entries."""
+    rows = len(row_index) - 1
     out = np.zeros(min(rows, max(int(slots), len(tiles), 1)), dtype=ROW_WORK)   # a row or more per segment
     n, words = ctypes.c_uint32(), (ctypes.c_uint32 * 3)()
     check(lib().nz_matvec_row_plan(descs.ctypes.data, tiles.ctypes.data if len(tiles) else None, len(tiles),
-                                   ctypes.cast(array, ctypes.c_void_p), len(weights), int(cols), int(element_size),
+                                   row_index.ctypes.data, rows, entries.ctypes.data, len(entries), int(cols),
                                    int(slots), float(first_weight), out.ctypes.data, len(out), ctypes.byref(n), words))
     return out[:n.value].copy(), tuple(words)
 

@@ -364,16 +364,16 @@ int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights,
 }
 
 int nz_matvec_row_plan(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
-                       const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, int element_size,
-                       uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
+                       const uint32_t* row_index, uint32_t n_rows, const uint32_t* entries, uint32_t n_entries,
+                       uint32_t cols, uint32_t slots, double first_weight, nz_row_work* out, uint32_t capacity,
                        uint32_t* n_segments, uint32_t* words) {
     return guarded([&] {
-        if (!frags || (!tiles && n_tiles) || !weights || (!out && capacity) || !n_segments || !words)
+        if (!frags || (!tiles && n_tiles) || !row_index || (!entries && n_entries) || (!out && capacity) ||
+            !n_segments || !words)
             nz::fail(nz::kInvalidArgument, "Null matvec plan argument.");
-        if (element_size != 2 && element_size != 4) nz::fail(nz::kInvalidArgument, "element_size must be 2 or 4.");
+        if (row_index[n_rows] != n_entries) nz::fail(nz::kInvalidArgument, "The row index ends at the entries' count.");
         const std::vector<nz_row_work> segs =
-            nz::plan_rows(frags, tiles, n_tiles, weights, n_weights, cols, static_cast<unsigned>(element_size), slots,
-                          first_weight);
+            nz::plan_rows(frags, tiles, n_tiles, row_index, n_rows, entries, cols, slots, first_weight);
         if (segs.size() > capacity) nz::fail(nz::kInvalidArgument, "Segment buffer is too small.");
         std::copy(segs.begin(), segs.end(), out);
         *n_segments = static_cast<uint32_t>(segs.size());

@@ -511,12 +511,14 @@ std::vector<nz_work> plan_work(const nz_frag_desc* frags, const nz_tile* tiles, 
 }
 
 std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
-                                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
-                                   unsigned element_size, uint32_t slots, double first_weight) {
+                                   const uint32_t* row_index, uint32_t n_rows, const uint32_t* entries, uint32_t cols,
+                                   uint32_t slots, double first_weight) {
     if (!(first_weight >= 1.0 && first_weight <= 16.0)) fail(kInvalidArgument, "first_weight must be in [1, 16].");
-    std::vector<uint32_t> row_index, entries;
-    plan_matvec(frags, tiles, n_tiles, weights, n_weights, cols, element_size, row_index, entries);
-    const uint32_t n_rows = static_cast<uint32_t>(row_index.size()) - 1;
+    if (row_index[0] != 0) fail(kInvalidArgument, "A row index starts at 0.");
+    for (uint32_t n = 0; n < n_rows; ++n)
+        if (row_index[n + 1] <= row_index[n]) fail(kInvalidArgument, "A row has no partial sum.");
+    for (uint32_t e = 0; e < row_index[n_rows]; ++e)
+        if (entries[e] / 2 >= n_tiles) fail(kInvalidArgument, "An entry names a tile past the list.");
     auto key = [&](uint32_t t) {
         const nz_frag_desc& f = frags[tiles[t].frag];
         return std::pair<uint64_t, uint32_t>(f.kind == NZ_KIND_RAW ? 0 : f.lut, f.kind);

@@ -95,15 +95,15 @@ void matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* ti
                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, unsigned element_size,
                   uint64_t store_bytes, nz_matvec_tile* out);
 
-// Row segments of the same product: one per workgroup, each owning whole
-// rows of the stacked output, with the shares of plan_work cut at rows.
-// Empty where some row's tiles are not adjacent in the launch order with one
+// Row segments of the same product from plan_matvec's row_index and entries:
+// one per workgroup, each owning whole rows of the stacked output, with the
+// shares of plan_work cut at rows. Empty where some row's tiles are not adjacent in the launch order with one
 // LUT and kind, or where cutting at rows would load a segment with over
-// kMaxRowExcess elements and a tenth more than its share. Fails where
-// plan_matvec would.
+// kMaxRowExcess elements and a tenth more than its share. Fails on entries
+// past the tiles or rows without one.
 std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
-                                   const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,
-                                   unsigned element_size, uint32_t slots, double first_weight);
+                                   const uint32_t* row_index, uint32_t n_rows, const uint32_t* entries, uint32_t cols,
+                                   uint32_t slots, double first_weight);
 
 // CPU emulation of the decode kernel over a packed buffer; writes words
 // into `out` (the output workspace image).

@@ -193,7 +193,7 @@ class HIPDecoder:
         order = sorted(fragment_indices, key=lambda i: (int(store.descs[i]["kind"]), int(store.descs[i]["lut"]), i))
         tiles = np.concatenate([store.fragment_tiles(i) for i in order])
         weights = tuple((int(offset), int(rows)) for _, offset, rows in members)
-        row_index, _ = _native.matvec_plan(store.descs, tiles, weights, cols, dtype.element_size)
+        row_index, entries = _native.matvec_plan(store.descs, tiles, weights, cols, dtype.element_size)
         # the kernel reads one record per tile (offsets, first column, partial position)
         records = _native.matvec_tiles(store.descs, tiles, weights, cols, dtype.element_size, store.buffer.numel())
         device = store.device
@@ -213,8 +213,7 @@ class HIPDecoder:
                 tensors.append(t)
                 launches.append((t.data_ptr(), len(group), long_codes))
         # the same product in one launch, where workgroups can own whole rows
-        row_segments, words = _native.matvec_row_plan(store.descs, tiles, weights, cols, dtype.element_size, slots,
-                                                      first_weight)
+        row_segments, words = _native.matvec_row_plan(store.descs, tiles, row_index, entries, cols, slots, first_weight)
         is_long = row_segments["kind"] == KIND_LONG
         row_groups = []
         for long_codes, group in enumerate((row_segments[~is_long], row_segments[is_long])):

@@ -42,8 +42,8 @@ def case_of(name, dtype):
 def test_row_segments_hold_every_sum_of_their_rows_once(name, slots, weight):
     dtype = torch.bfloat16
     base, descs, tiles, weights, cols = case_of(name, dtype)
-    segments, words = _native.matvec_row_plan(descs, tiles, weights, cols, 2, slots, weight)
-    row_index, _ = _native.matvec_plan(descs, tiles, weights, cols, 2)
+    row_index, entries = _native.matvec_plan(descs, tiles, weights, cols, 2)
+    segments, words = _native.matvec_row_plan(descs, tiles, row_index, entries, cols, slots, weight)
     records = _native.matvec_tiles(descs, tiles, weights, cols, 2, base.size)
     assert len(segments) and segments["row0"][np.argsort(segments["row0"])][0] == 0
     owned = np.zeros(len(row_index) - 1, int)
@@ -68,7 +68,9 @@ def test_row_segments_hold_every_sum_of_their_rows_once(name, slots, weight):
 def test_no_row_plan_where_codebooks_change_inside_rows():
     w, enc, offset = encoded_case("nzm1", torch.bfloat16)     # chunks of 9.14 rows, two codebooks in turn
     _, descs, tiles = enc.host_image()
-    segments, _ = _native.matvec_row_plan(descs, launch_order(descs, tiles), [(offset, w.shape[0])], w.shape[1], 2, 512)
+    tiles = launch_order(descs, tiles)
+    plan = _native.matvec_plan(descs, tiles, [(offset, w.shape[0])], w.shape[1], 2)
+    segments, _ = _native.matvec_row_plan(descs, tiles, *plan, w.shape[1], 512)
     assert not len(segments)
 
 
@@ -76,10 +78,10 @@ def run_rows(base, descs, tiles, dtype, weights, cols, x, biases, slots, first_w
     """The one-launch form's outputs, whose buffers start as NaN words."""
     spec, batch = DTYPES[dtype], x.shape[0]
     es, reorder = spec.element_size, int(spec.bit_reorder)
-    segments, words = _native.matvec_row_plan(descs, tiles, weights, cols, es, slots, first_weight)
+    row_index, entries = _native.matvec_plan(descs, tiles, weights, cols, es)
+    segments, words = _native.matvec_row_plan(descs, tiles, row_index, entries, cols, slots, first_weight)
     need = words[min(batch - 1, 2)]
     assert len(segments) and need <= _native.lib().nz_matvec_row_words(es, batch)
-    row_index, _ = _native.matvec_plan(descs, tiles, weights, cols, es)
     records = _native.matvec_tiles(descs, tiles, weights, cols, es, base.size)
     device = [torch.from_numpy(a.view(np.uint8).copy()).cuda() for a in (base, descs, records, row_index)]
     ys = [torch.full((batch * rows * es,), 0xFF, dtype=torch.uint8, device="cuda").view(dtype).view(batch, rows)
