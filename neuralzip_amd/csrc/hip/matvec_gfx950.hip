@@ -248,6 +248,10 @@ constexpr uint32_t early_rounds() { return BT == 1 ? 2 : 1; }
 // round per 64 vectors. What holds for a whole round (all vectors inside the
 // tile, all on one side of the row split, none at all) is decided by scalar
 // branches; only a round that the tile's end or the split cuts masks lanes.
+// Either way a vector's products are summed from zero and then added to the
+// lane's sum. (Chained through the lane's sum instead, 16 fp32 products in a
+// row, 28672 x 4096 bf16 took 41.9 us against 42.1, and fp32 products of 4096
+// to 14336 columns had up to a tenth more error.)
 template <int ES, bool REORDER, bool LONG, int BT>
 __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES, LONG>& d, const uint8_t* stage,
                                               const RowSpan& rs, const Activations<BT>& x, uint32_t cols,
@@ -276,7 +280,7 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
         if (ti.s0 == 0 && min(ti.s1, rs.split) >= (r + 1) * kSpan) {   // every vector inside the tile's first row
             asm volatile("");
 #pragma unroll
-            for (int b = 0; b < BT; ++b) p.acc[0][b] = dot_vector<ES, REORDER>(v, xv[b], p.acc[0][b]);
+            for (int b = 0; b < BT; ++b) p.acc[0][b] += dot_vector<ES, REORDER>(v, xv[b], 0.0f);
         } else {
             asm volatile("");
             // staged bytes outside the tile are the neighbours': keep them out of the sums
