@@ -14,8 +14,7 @@
 //     and tile decode (tile_decode.h). Instead of storing the merged words, a
 //     wavefront multiplies them by the activations with v_dot2 (products
 //     accumulated in fp32) and reduces its lanes with DPP. A tile holds at
-//     most 2048 elements (raw ones; coded ones fewer), so with cols >= 2048
-//     it touches at most two rows;
+//     most 2048 elements, so with cols >= 2048 it touches at most two rows;
 //     the wavefront writes one partial sum per (row slot, activation row).
 //   * nz_matvec_rows_kernel: the same for plans whose workgroups own whole
 //     rows, which add up their rows' partial sums in LDS: the whole product

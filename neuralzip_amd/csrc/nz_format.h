@@ -35,13 +35,14 @@
 
 #define NZ_WINDOW_BITS 64
 #define NZ_WAVE 64
-// Max exponent bytes staged per tile (16-bit words): three merge rounds of 64
+// Max exponent bytes staged per tile (16-bit words): four merge rounds of 64
 // lanes x 8 elements. 64 windows of N(0, std^2) bf16 weights hold about 1600
-// elements; with 2048 (four rounds) most tiles ran a fourth round for a few
-// lanes and all tiles issued its loads and stores. 28672 x 4096 bf16 product
-// 44.9 -> 43.3 us, 4096 x 14336 fp16 42.4 -> 38.4, 277 M bf16 elements decoded
-// 168.5 -> 167.7; uniform weights, 2048 elements per 64 windows, 44.4 -> 44.2.
-#define NZ_TILE_OUT 1536
+// elements, of uniform ones 2048. A limit of 1536 (three rounds) spares the
+// former the fourth round's few lanes (28672 x 4096 bf16 product 41.6 us
+// against 43.8), but takes lanes from codes under two bits: the same product
+// with 90 % zeros 57.2 against 47.8, ternary 46.2 against 39.5; 14.9 M ternary
+// weights decoded 10.6 against 9.1, 277 M equal ones 287 against 274.
+#define NZ_TILE_OUT 2048
 #define NZ_TILE_OUT32 1024        // the same for 32-bit words
 #define NZ_RAW_TILE 2048          // elements per tile of a raw fragment
 #define NZ_TILE_ALIGN 64          // Huffman tiles end on multiples of this many output elements

@@ -1,46 +1,58 @@
-"""Tiles of 16-bit words stage at most 1536 elements (three merge rounds):
-sizes around one, two and three rounds and around a second tile, with codes
-short enough for the limit to bind and long enough for 64 windows to bind."""
+"""Tiles stage at most 2048 elements of 16-bit words and 1024 of 32-bit ones
+(four merge rounds), the elements of its first vector ahead of a tile's first
+one included: sizes around the rounds and around a second tile, at aligned and
+odd places of the workspace, with codes short enough for the limit to bind and
+long enough for 64 windows to bind."""
 import numpy as np
 import pytest
 import torch
 
 from neuralzip_amd import _native
+from neuralzip_amd.dtypes import DTYPES
 from nz_helpers import Encoded, singleton_header
 from test_layout_emulator import emulate_case
 
+LIMIT = {torch.bfloat16: 2048, torch.float16: 2048, torch.float32: 1024}
+OFFSETS = (8, 3, 7)
 
-def words_of(kind, n):
+
+def words_of(kind, n, dtype):
     g = torch.Generator().manual_seed(n)
     if kind == "limit":     # one bit per exponent or so
-        return torch.where(torch.rand(n, generator=g) < 0.9, 0.5, 0.01).bfloat16()
-    return torch.randn(n, generator=g).mul(0.02).bfloat16()
+        return torch.where(torch.rand(n, generator=g) < 0.9, 0.5, 0.01).to(dtype)
+    return torch.randn(n, generator=g).mul(0.02).to(dtype)
 
 
-SIZES = (1, 511, 513, 1023, 1025, 1535, 1536, 1537, 1600, 3071, 3073, 10001)
+SIZES = (1, 511, 513, 1023, 1025, 1535, 1536, 1537, 1600, 2047, 2048, 2049, 3071, 3073, 4095, 4097, 10001)
 
 
-def case_of(kind, n):
-    raw = words_of(kind, n).view(torch.uint8).numpy().copy()
-    book = _native.Codebook(singleton_header(words_of(kind, 40000).view(torch.uint8).numpy(), torch.bfloat16, prior=1))
-    return [(raw, torch.bfloat16, 1 << 20, [0], 8)], {0: book}
+def case_of(kind, n, dtype, offset):
+    raw = words_of(kind, n, dtype).view(torch.uint8).numpy().copy()
+    book = _native.Codebook(singleton_header(words_of(kind, 40000, dtype).view(torch.uint8).numpy(), dtype, prior=1))
+    return [(raw, dtype, 1 << 20, [0], offset)], {0: book}
 
 
+@pytest.mark.parametrize("offset", OFFSETS)
+@pytest.mark.parametrize("dtype", sorted(LIMIT, key=str))
 @pytest.mark.parametrize("kind", ["limit", "windows"])
-@pytest.mark.parametrize("n", SIZES)
-def test_tiles_hold_at_most_three_rounds(kind, n):
-    tensors, books = case_of(kind, n)
-    _, _, tiles = Encoded(tensors, books).host_image()
-    assert tiles["n_out"].max() <= 1536 and tiles["n_out"].astype(int).sum() == n
-    if kind == "limit" and n > 1536:
-        assert tiles["n_out"].max() > 1536 - 64
-    emulate_case(tensors, books, torch.bfloat16)
+def test_tiles_hold_at_most_four_rounds(kind, dtype, offset):
+    vector, limit = 16 // DTYPES[dtype].element_size, LIMIT[dtype]
+    for n in SIZES:
+        tensors, books = case_of(kind, n, dtype, offset)
+        _, _, tiles = Encoded(tensors, books).host_image()
+        ahead = (offset + tiles["out0"].astype(int)) % vector
+        assert (ahead + tiles["n_out"]).max() <= limit and tiles["n_out"].astype(int).sum() == n
+        if kind == "limit" and n > limit + 64:     # the limit binds, but for the line its end is cut back to
+            assert tiles["n_out"].max() > limit - 64
+        emulate_case(tensors, books, dtype)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", sorted(LIMIT, key=str))
 @pytest.mark.parametrize("kind", ["limit", "windows"])
 @pytest.mark.parametrize("n", SIZES)
-def test_tiles_of_three_rounds_decode(kind, n):
+def test_tiles_of_four_rounds_decode(kind, n, dtype):
     from test_gpu_decode import check_case
-    tensors, books = case_of(kind, n)
-    check_case(tensors, books, torch.bfloat16)
+    for offset in OFFSETS:
+        tensors, books = case_of(kind, n, dtype, offset)
+        check_case(tensors, books, dtype)
