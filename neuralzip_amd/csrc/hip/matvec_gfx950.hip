@@ -217,6 +217,7 @@ __device__ __forceinline__ void fetch_x(const Activations<BT>& x, const RowSpan&
         asm volatile("");
 #pragma unroll
         for (uint32_t r = R0; r < R1; ++r) {
+            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * Geometry<ES>::V) break;
             const uint32_t a = at + r * NZ_WAVE * 16u;
 #pragma unroll
             for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], min(a, a - cols * ES));
@@ -224,9 +225,11 @@ __device__ __forceinline__ void fetch_x(const Activations<BT>& x, const RowSpan&
     } else {
         asm volatile("");
 #pragma unroll
-        for (uint32_t r = R0; r < R1; ++r)
+        for (uint32_t r = R0; r < R1; ++r) {
+            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * Geometry<ES>::V) break;
 #pragma unroll
             for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], at + r * NZ_WAVE * 16u);
+        }
     }
 }
 
@@ -263,7 +266,8 @@ __device__ __forceinline__ void multiply_tile(const TileInfo& ti, const Fetch<ES
 #pragma unroll
     for (uint32_t r = 0; r < G::kRounds; ++r) {
         if (ti.s1 <= r * kSpan) continue;
-        if (BT > 1 && r + 1 < G::kRounds) fetch_x_round<ES, BT>(x, rs, ti, cols, lane, r + 1, r % 2 ? early[0] : late[0]);
+        if (BT > 1 && r + 1 < G::kRounds && !(late_round<ES>(r + 1) && ti.s1 <= (r + 1) * kSpan))
+            fetch_x_round<ES, BT>(x, rs, ti, cols, lane, r + 1, r % 2 ? early[0] : late[0]);
         const uint4* xv = BT == 1 ? (r < E ? early[r % E] : late[(r - E) % (G::kRounds - E)]) : r % 2 ? late[0] : early[0];
         const uint32_t g = (lane + NZ_WAVE * r) * V;
         const uint8_t* at = stage + NZ_STAGE_ORIGIN + g;
@@ -340,7 +344,7 @@ __device__ __forceinline__ void huffman_segment(const uint8_t* base, const nz_ma
         const TileInfo nxt = tile_record<ES>(base, tiles, more ? tn : t, cols, rn);
         Fetch<ES, LONG> fn;
         const uint32_t after = more ? claim(counter) : n;
-        fetch_raw<ES, LONG>(cur, lane, fc);
+        fetch_raw<ES, LONG, true>(cur, lane, fc);
         uint4 early[early_rounds<BT>()][BT];
         fetch_x<ES, BT, 0, early_rounds<BT>()>(x, rs, cur, cols, lane, early);
         const LaneDecode l = open_tile<ES, LONG>(cur, fc, stage, lane);

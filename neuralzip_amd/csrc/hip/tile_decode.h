@@ -238,14 +238,26 @@ __device__ __forceinline__ void fetch_bits(const TileInfo& ti, uint32_t lane, Fe
     }
 }
 
-// The part used only after the decode: raw lanes.
-template <int ES, bool LONG>
+// Merge rounds that a tile of 16-bit words may not reach: 64 windows hold
+// anything from a few hundred elements (fp16: about 740) to the limit. The
+// fused kernel leaves their loads out by scalar branches: 4096 x 14336 fp16
+// took 41.9 us with the loads of all rounds in every tile and 32.8 without,
+// for four activation rows 71.7 and 56.1; 28672 x 4096 bf16 (tiles of 1600,
+// all four rounds) 43.8 and 43.0. 32-bit words reach their limit but with
+// codes over four bits, and the branches alone cost them 2 %.
+template <int ES>
+constexpr bool late_round(uint32_t r) { return ES == 2 && r >= 2; }
+
+// The part used only after the decode: raw lanes. With TRIM, rounds that the
+// tile does not reach (late_round) are left out by a scalar branch.
+template <int ES, bool LONG, bool TRIM = false>
 __device__ __forceinline__ void fetch_raw(const TileInfo& ti, uint32_t lane, Fetch<ES, LONG>& d) {
     using G = Geometry<ES>;
     const uint32_t span = ti.nv * G::V;   // lane bytes covering the tile's vectors
     const rsrc_t lanes = make_rsrc(ti.lanes, ES == 2 ? span : 2 * ti.stride + span);
 #pragma unroll
     for (uint32_t r = 0; r < G::kRounds; ++r) {
+        if (TRIM && late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * G::V) break;
         const uint32_t at = (lane + NZ_WAVE * r) * G::V;
         if (ES == 2) {
             const v2u v = __builtin_amdgcn_raw_buffer_load_b64(lanes, at, 0, 0);

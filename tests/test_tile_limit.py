@@ -56,3 +56,25 @@ def test_tiles_of_four_rounds_decode(kind, n, dtype):
     for offset in OFFSETS:
         tensors, books = case_of(kind, n, dtype, offset)
         check_case(tensors, books, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", sorted(LIMIT, key=str))
+@pytest.mark.parametrize("elements", [8, 512, 1016, 1024, 1032, 1528, 1536, 1544, 2040, 2048])
+def test_products_of_tiles_that_end_around_each_round(elements, dtype, batch):
+    """One tile per chunk of `elements` (two where 32-bit words exceed their
+    limit), across the ends of rows, both ways of adding the tiles up."""
+    from test_matvec import check_product, run_matvec
+    from test_row_products import run_rows
+    rows, cols = 9, 2048
+    w = words_of("limit", rows * cols, dtype).view(rows, cols)
+    raw = w.view(torch.uint8).numpy().reshape(-1).copy()
+    books = {0: _native.Codebook(singleton_header(raw, dtype, prior=1))}
+    base, descs, tiles = Encoded([(raw, dtype, elements, [0] * -(-w.numel() // elements), 64)], books).host_image()
+    assert elements > LIMIT[dtype] or tiles["n_out"][0] == elements
+    x = torch.randn(batch, cols, generator=torch.Generator().manual_seed(batch)).to(dtype)
+    (two,) = run_matvec(base, descs, tiles, dtype, [(64, rows)], cols, x, calls=1)
+    check_product(two[0], w, x, None, dtype)
+    (one,) = run_rows(base, descs, tiles, dtype, [(64, rows)], cols, x, [None], 64, 1.0)
+    assert torch.equal(one.view(torch.uint8), two[0].view(torch.uint8))
