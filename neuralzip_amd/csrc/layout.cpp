@@ -256,8 +256,9 @@ void pack_fragment(const Fragment& f, uint8_t* dst, uint64_t offset, uint64_t lu
 }
 
 constexpr uint64_t kMinTilesPerGroup = 16;
-// Elements that a row segment may have above its share: a workgroup takes
-// about 2.5 us for as many, less than the reduce launch it saves (7 us).
+// Elements that a row segment may have above the largest segment of a plan cut
+// at tiles: a workgroup takes about 2.5 us for as many, less than the reduce
+// launch it saves (7 us).
 constexpr double kMaxRowExcess = 16384;
 constexpr size_t kXcds = 8;   // MI355X: accelerator dies, each with its own L2
 
@@ -552,6 +553,18 @@ std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* til
     // the weights of plan_work
     const bool paired = first_weight != 1.0 && total == slots && slots % 2 == 0 && !(any_long && any_other);
     auto weight = [&](uint64_t b) { return paired && b < slots / 2 ? first_weight : 1.0; };
+    // Rows are few and long, or change codebook often, where whole rows would
+    // keep a workgroup busy long after plan_work's had ended (1 x 1048576: one
+    // workgroup for all against 41 of 25600), or run after all the others
+    // (more segments than slots). Those products take two launches.
+    const std::vector<nz_work> cut = plan_work(frags, tiles, n_tiles, slots);
+    if (total > std::max<uint64_t>(slots, cut.size())) return {};
+    double largest = 0;   // elements of the largest of them, raw ones at half weight
+    for (const nz_work& s : cut) {
+        double n = 0;
+        for (uint32_t t = s.tile0; t < s.tile1; ++t) n += nz_tile_elements(tiles[t].counts);
+        largest = std::max(largest, s.kind == NZ_KIND_RAW ? 0.5 * n : n);
+    }
     std::vector<nz_row_work> out;
     for (size_t i = 0; i < runs.size(); ++i) {
         const nz_row_work& run = runs[i];
@@ -567,8 +580,10 @@ std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* til
             const uint32_t end = j + 1 == parts ? run.row1
                                  : std::min<uint32_t>(std::max(want, row + 1),
                                                       run.row1 - static_cast<uint32_t>(parts - j - 1));
-            const double excess = (end - row) - rows * weight(base + j) / weights_sum;   // rows above the exact share
-            if (excess * cols > kMaxRowExcess && excess > 0.1 * (end - row)) return {};
+            const double n = (run.kind == NZ_KIND_RAW ? 0.5 : 1.0) * (end - row) * cols;
+            // weights of 1 on average; at most 1.4 us were lost where all were 1
+            const double excess = n - largest * std::max(1.0, paired ? 2 * weight(base + j) / (1 + first_weight) : 1.0);
+            if (excess > kMaxRowExcess && excess > 0.1 * n) return {};
             out.push_back({first(row), last(end - 1) + 1, tiles[first(row)].frag, run.kind, row, end, row_index[row],
                            row_index[end] - row_index[row]});
             row = end;

@@ -97,10 +97,12 @@ void matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* ti
 
 // Row segments of the same product from plan_matvec's row_index and entries:
 // one per workgroup, each owning whole rows of the stacked output, with the
-// shares of plan_work cut at rows. Empty where some row's tiles are not adjacent in the launch order with one
-// LUT and kind, or where cutting at rows would load a segment with over
-// kMaxRowExcess elements and a tenth more than its share. Fails on entries
-// past the tiles or rows without one.
+// shares of plan_work cut at rows. Empty where some row's tiles are not
+// adjacent in the launch order with one LUT and kind, where a segment would
+// get over kMaxRowExcess elements and a tenth more than plan_work's largest
+// (each against its weight), or where there would be more segments than slots
+// and than plan_work makes. Fails on entries past the tiles or rows without
+// one.
 std::vector<nz_row_work> plan_rows(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles,
                                    const uint32_t* row_index, uint32_t n_rows, const uint32_t* entries, uint32_t cols,
                                    uint32_t slots, double first_weight);

@@ -74,6 +74,54 @@ def test_no_row_plan_where_codebooks_change_inside_rows():
     assert not len(segments)
 
 
+def plain_tiles(rows, cols, elements, chunk=None, books=1, kind=_native.KIND_SHORT):
+    """Descriptors and launch-ordered tiles of a rows x cols weight in chunks
+    whose codebooks take turns: what the planners read of them."""
+    total, chunk = rows * cols, chunk or rows * cols
+    starts = np.arange(0, total, chunk)
+    descs = np.zeros(len(starts), _native.FRAG_DESC)
+    descs["kind"], descs["out"], descs["lut"] = kind, starts, np.arange(len(starts)) % books * 65536
+    tiles = []
+    for f, start in enumerate(starts):
+        size = min(chunk, total - start)
+        t = np.zeros(-(-size // elements), _native.TILE)
+        t["frag"], t["out0"] = f, np.arange(0, size, elements)
+        t["n_out"] = np.minimum(elements, size - t["out0"].astype(int))
+        tiles.append(t)
+    return descs, launch_order(descs, np.concatenate(tiles))
+
+
+@pytest.mark.parametrize("rows,cols,elements,chunk,books,slots,whole", [
+    # few rows of very many columns: whole rows would be a few workgroups of a million elements
+    (1, 1 << 20, 1600, None, 1, 512, False), (4, 131072, 1600, None, 1, 512, False),
+    (64, 65536, 1024, None, 1, 512, False), (64, 49152, 1600, None, 1, 512, False),
+    # codebooks that change after every few rows: more row segments than the device runs at once,
+    # as many as it runs, and (uneven) a few fewer
+    (34 * 32, 4096, 1600, 131072, 2, 32, False), (32 * 32, 4096, 1600, 131072, 2, 32, True),
+    (20 * 32, 4096, 1600, 131072, 2, 32, False), (34 * 2, 4096, 1600, 8192, 2, 32, False),
+    # short and long rows that divide evenly enough
+    (6144, 4096, 1600, None, 1, 512, True), (4096, 14336, 704, None, 1, 512, True),
+    (8192, 28672, 1600, None, 1, 512, True), (300, 28672, 1600, None, 1, 512, True),
+    (40, 8192, 1600, None, 1, 512, True), (1, 16384, 1600, None, 1, 512, True)])
+def test_row_segments_are_hardly_larger_than_those_cut_at_tiles(rows, cols, elements, chunk, books, slots, whole):
+    """With a row plan, no segment has over 16384 elements and a tenth more
+    than the largest of nz_plan_work's, and there are no more of them than run at once; what would
+    break that has none (and takes two launches)."""
+    elements = elements // 64 * 64
+    descs, tiles = plain_tiles(rows, cols, elements, chunk, books)
+    row_index, entries = _native.matvec_plan(descs, tiles, [(0, rows)], cols, 2)
+    sizes = tiles["n_out"].astype(int)
+    for first_weight in (1.0, 1.75):
+        segments, _ = _native.matvec_row_plan(descs, tiles, row_index, entries, cols, slots, first_weight)
+        cut = _native.plan_work(descs, tiles, slots, first_weight)
+        assert bool(len(segments)) == whole
+        if whole:
+            largest = max(sizes[s["tile0"]:s["tile1"]].sum() for s in cut)
+            most = (segments["row1"] - segments["row0"]).astype(int).max() * cols
+            assert most <= max(largest + 16384, largest / 0.9)
+            assert len(segments) <= max(slots, len(cut))
+
+
 def run_rows(base, descs, tiles, dtype, weights, cols, x, biases, slots, first_weight):
     """The one-launch form's outputs, whose buffers start as NaN words."""
     spec, batch = DTYPES[dtype], x.shape[0]
