@@ -318,7 +318,7 @@ int nz_matvec_reduce(const uint32_t* row_index, const nz_matvec_weight* weights,
  * nz_matvec_plan took and gave them, slots and first_weight as for
  * nz_plan_work. *n_segments receives 0 where the product has no such
  * plan: a row in tiles of two codebooks or of separate places of the launch
- * order, rows so long that a segment would get over 16384 elements and a
+ * order, rows so long that a segment would get over 24576 elements and a
  * tenth more than nz_plan_work's largest, or codebooks that change between
  * rows so often that there would be more segments than slots (and than
  * nz_plan_work makes). words[i] (i = 0, 1, 2) receives the LDS words that the

@@ -257,9 +257,13 @@ void pack_fragment(const Fragment& f, uint8_t* dst, uint64_t offset, uint64_t lu
 
 constexpr uint64_t kMinTilesPerGroup = 16;
 // Elements that a row segment may have above the largest segment of a plan cut
-// at tiles: a workgroup takes about 2.5 us for as many, less than the reduce
-// launch it saves (7 us).
-constexpr double kMaxRowExcess = 16384;
+// at tiles. The reduce launch it saves takes about 5 us; a workgroup takes 1.5
+// us for 16384 bf16 elements when it runs alone, 2.8 for fp32 ones or beside
+// another on its compute unit, so rows pay up to about 29000. Measured (us, rows
+// against two launches): 64 x 49152 bf16, 23552 above, 9.9 and 12.9; 64 x 65536
+// fp32, 49152 above, 16.1 and 13.0; 4 x 131072 bf16, 105472 above, 17.4 and 12.9;
+// 1 x 1048576 bf16 109 and 37.
+constexpr double kMaxRowExcess = 24576;
 constexpr size_t kXcds = 8;   // MI355X: accelerator dies, each with its own L2
 
 void check_matvec_group(const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, unsigned element_size) {
