@@ -229,6 +229,7 @@ void nz_decode_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __re
     // claims start behind those. Its bits are requested beside the LUT, so
     // that a workgroup with few tiles waits for both at once.
     const uint32_t n = seg.tile1 - seg.tile0;
+    if (n == 0) return;   // an empty segment has no first tile to describe
     if (threadIdx.x == 0) lds.claim[0] = first_early(ES) ? WAVES * NZ_WAVE : 0;
     LutCopy<REORDER, WAVES * NZ_WAVE> lut;
     lut.fetch(base + frags[seg.lut_frag].lut, threadIdx.x);

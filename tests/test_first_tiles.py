@@ -32,3 +32,27 @@ def test_workgroups_of_few_tiles(tiles, dtype, flags):
     n = low - 1 + low % 2
     assert count(n) == tiles
     check_case(tensors(n), {0: book}, dtype, slots=1, interleaved=True, flags=flags)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flags", [0, _native.DECODE_HALF_GROUPS, _native.DECODE_CACHED_STORES])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_empty_segments_decode_nothing(dtype, flags, monkeypatch):
+    """Segments without tiles, which a caller's own plan may hold: before,
+    between and behind the others, the last past the end of the tile list."""
+    plan_work = _native.plan_work
+
+    def with_empty_segments(descs, tiles, slots):
+        segments = plan_work(descs, tiles, slots)
+        empty = segments[:1].copy()
+        parts = []
+        for at in (0, segments["tile1"][0], len(tiles)):
+            empty["tile0"] = empty["tile1"] = at
+            parts.append(empty.copy())
+        return np.concatenate([parts[0], segments[:1], parts[1], segments[1:], parts[2]])
+
+    monkeypatch.setattr(_native, "plan_work", with_empty_segments)
+    words = (torch.randn(50001, generator=torch.Generator().manual_seed(2)) * 0.02).to(dtype)
+    raw = words.view(torch.uint8).numpy().copy()
+    check_case([(raw, dtype, 20000, [0, -1, 0], 3)], {0: _native.Codebook(singleton_header(raw, dtype))}, dtype, slots=4,
+               flags=flags)
