@@ -293,7 +293,8 @@ int nz_matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* 
  * elements with x (device, batch x cols in the weights' dtype, 1 <= batch
  * <= NZ_MATVEC_MAX_BATCH) summed per row they touch, in
  * partials[position * batch + b] (device fp32, room for 2 * n_tiles * batch
- * values; positions as in nz_matvec_plan, from each tile's record). `tiles`
+ * values, past which nothing is stored; positions as in nz_matvec_plan, from
+ * each tile's record). `tiles`
  * is a device copy of nz_matvec_tiles' records for `base`
  * (the packed buffer they were checked against); `frags` gives each
  * segment's LUT. One call per codebook kind (long_codes) of the tiles.

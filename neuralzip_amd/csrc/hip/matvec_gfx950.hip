@@ -142,12 +142,13 @@ __device__ __forceinline__ TileInfo tile_record(const uint8_t* base, const nz_ma
 }
 
 // Where partial sums go: the product's array in device memory, for the
-// reduce launch ...
+// reduce launch (two positions per tile of the product; records of a larger
+// one store nothing past them) ...
 struct GlobalSums {
     float* partials;
-    uint32_t batch;
+    uint32_t batch, n_tiles;
     __device__ __forceinline__ void put(uint32_t entry, int b, float v) const {
-        if (b < static_cast<int>(batch)) partials[entry * batch + b] = v;
+        if (b < static_cast<int>(batch) && entry / 2 < n_tiles) partials[entry * batch + b] = v;
     }
 };
 
@@ -453,7 +454,7 @@ template <int ES, bool REORDER, bool LONG, int BT>
 __global__ __launch_bounds__(matvec_threads<BT>()) __attribute__((amdgpu_waves_per_eu(BT <= 2 ? 8 : 6)))
 void nz_matvec_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __restrict__ frags,
                       const nz_matvec_tile* __restrict__ tiles, const nz_work* __restrict__ segs, uint32_t cols,
-                      const uint8_t* __restrict__ xp, uint32_t batch, float* __restrict__ partials) {
+                      const uint8_t* __restrict__ xp, uint32_t batch, float* __restrict__ partials, uint32_t n_tiles) {
     __shared__ __align__(16) GroupLds<ES, matvec_waves<BT>()> lds;
     const uint32_t lane = lane_index();
     const nz_work seg = segs[blockIdx.x];
@@ -466,7 +467,7 @@ void nz_matvec_kernel(const uint8_t* __restrict__ base, const nz_frag_desc* __re
     }
     __syncthreads();
     run_segment<ES, REORDER, LONG, BT>(base, tiles + seg.tile0, seg.tile1 - seg.tile0, seg.kind, lds, lane, cols, x,
-                                       GlobalSums{partials, batch});
+                                       GlobalSums{partials, batch, n_tiles});
 }
 
 // fp32 to the weight's dtype, rounding to nearest even.
@@ -610,7 +611,7 @@ hipError_t launch_matvec(const void* base, const void* frags, const void* tiles,
     hipLaunchKernelGGL((nz_matvec_kernel<ES, REORDER, LONG, BT>), dim3(n_segs), dim3(matvec_threads<BT>()), 0, stream,
                        static_cast<const uint8_t*>(base), static_cast<const nz_frag_desc*>(frags),
                        static_cast<const nz_matvec_tile*>(tiles), static_cast<const nz_work*>(segs), cols,
-                       static_cast<const uint8_t*>(x), batch, partials);
+                       static_cast<const uint8_t*>(x), batch, partials, n_tiles);
     return hipGetLastError();
 }
 
@@ -675,8 +676,9 @@ bool layout_ok(int element_size, int bit_reorder, char* message, size_t message_
 }  // namespace
 
 // Partial sums of one launch (one codebook kind) of a product's tiles:
-// writes partials[(2 * t + slot) * batch + b] for every tile t the segments
-// cover. `tiles` are nz_matvec_tile records the host checked against `base`.
+// writes partials[(entry + slot) * batch + b] for every tile the segments
+// cover, `entry` from its record, below position 2 * n_tiles. `tiles` are
+// nz_matvec_tile records the host checked against `base`.
 extern "C" int nz_hip_matvec_launch(const void* base, const void* frags, const void* tiles, const void* segs,
                                     uint32_t n_segs, int element_size, int bit_reorder, int long_codes, uint32_t cols,
                                     const void* x, uint32_t batch, float* partials, uint32_t n_tiles, void* stream,

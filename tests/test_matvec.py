@@ -345,6 +345,36 @@ def test_matvec_long_codes():
     check_product(first, w, x, None, torch.bfloat16)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 2, 3])
+def test_partial_sums_end_at_the_tiles_the_caller_named(batch):
+    """nz_matvec_launch with records of a larger product than `n_tiles` says:
+    positions from 2 * n_tiles on (here still inside the buffer) keep what
+    they held, those before get the sums of the whole product's launch."""
+    w, enc, offset = encoded_case("huff0", torch.bfloat16)
+    base, descs, tiles = enc.host_image()
+    tiles = launch_order(descs, tiles)
+    rows, cols = w.shape
+    records = _native.matvec_tiles(descs, tiles, [(offset, rows)], cols, 2, len(base))
+    segments = _native.plan_work(descs, tiles, 16)
+    dev = [torch.from_numpy(a.view(np.uint8).copy()).cuda() for a in (base, descs, records, segments)]
+    x = torch.randn(batch, cols, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).cuda()
+
+    def sums(n_tiles):
+        partials = torch.full((2 * len(tiles) * batch,), float("nan"), device="cuda")
+        _native.matvec_launch(*(d.data_ptr() for d in dev), len(segments), 2, 1, 0, cols, x.data_ptr(), batch,
+                              partials.data_ptr(), n_tiles, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return partials.cpu().view(torch.int32)
+
+    whole, named = sums(len(tiles)), len(tiles) // 3
+    part = sums(named)
+    cut = 2 * named * batch
+    assert int(records["entry"].max()) >= 2 * named
+    assert torch.equal(part[:cut], whole[:cut])
+    assert torch.isnan(part[cut:].view(torch.float32)).all()
+
+
 def grouped_case(dtype):
     """Three weights sharing x (rows stacked in workspace order, a raw chunk
     and two codebooks among them): (weights, base, descs, tiles, x, biases,
