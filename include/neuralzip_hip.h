@@ -337,9 +337,9 @@ uint32_t nz_matvec_row_words(int element_size, uint32_t batch);
 /* The product over row segments of one codebook kind (long_codes), complete:
  * weights[k].y as nz_matvec_launch and nz_matvec_reduce leave it, the same
  * bits. `words`: the plan's for this batch, checked against
- * nz_matvec_row_words. row_index is a device copy of nz_matvec_plan's.
- * Asynchronous on `stream`. No counterpart in the reference (see
- * nz_matvec_plan). */
+ * nz_matvec_row_words. row_index is a device copy of nz_matvec_plan's. Rows
+ * of the segments past the weights' are not stored. Asynchronous on `stream`.
+ * No counterpart in the reference (see nz_matvec_plan). */
 int nz_matvec_rows(const void* base, const nz_frag_desc* frags, const nz_matvec_tile* tiles,
                    const nz_row_work* segments, uint32_t n_segments, uint32_t words, int element_size,
                    int bit_reorder, int long_codes, const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols,

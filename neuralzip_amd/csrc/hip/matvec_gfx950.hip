@@ -596,6 +596,7 @@ void nz_matvec_rows_kernel(const uint8_t* __restrict__ base, const nz_frag_desc*
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < rows * batch; i += matvec_threads<BT>()) {
         const uint32_t b = i / rows, row = i - b * rows, n = seg.row0 + row;
+        if (n >= g.total_rows) continue;   // segments of a larger product
         const uint32_t w = weight_of(g, n), local = n - g.row_base[w];
         const float add = row_bias<ES, REORDER>(g, w, local);
         const float sum = sum_in_order(lds.words[row], lds.words[row + 1],

@@ -168,6 +168,33 @@ def test_one_launch_gives_the_bits_of_two(name, dtype, batch):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), f"weight {k}, {slots} slots"
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dropped", [1, 7, 36, 37])
+def test_rows_past_the_weights_are_left_alone(dropped):
+    """Row segments of a larger product than the weights say: rows past
+    theirs (here still inside the output) keep what they held."""
+    base, descs, tiles, weights, cols = case_of("odd-rows", torch.bfloat16)
+    rows = weights[0][1] - dropped
+    row_index, entries = _native.matvec_plan(descs, tiles, weights, cols, 2)
+    segments, words = _native.matvec_row_plan(descs, tiles, row_index, entries, cols, 64)
+    records = _native.matvec_tiles(descs, tiles, weights, cols, 2, base.size)
+    dev = [torch.from_numpy(a.view(np.uint8).copy()).cuda() for a in (base, descs, records, segments, row_index)]
+    x = torch.randn(1, cols, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).cuda()
+
+    def product(named):
+        y = torch.full((sum(r for _, r in weights),), float("nan"), dtype=torch.bfloat16, device="cuda")
+        array = _native.matvec_weights([(0, named, y.data_ptr(), None)])
+        _native.check(_native.lib().nz_matvec_rows(
+            *(d.data_ptr() for d in dev[:4]), len(segments), words[0], 2, 1, 0, array, 1, cols, x.data_ptr(), 1,
+            dev[4].data_ptr(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return y.cpu()
+
+    whole, part = product(sum(r for _, r in weights)), product(rows)
+    assert torch.isfinite(whole.float()).all() and torch.isnan(part[rows:].float()).all()
+    assert torch.equal(part[:rows].view(torch.int16), whole[:rows].view(torch.int16))
+
+
 def test_row_launch_refuses_segments_larger_than_the_lds():
     words = _native.lib().nz_matvec_row_words(2, 1)
     assert 1000 < words < 40960
