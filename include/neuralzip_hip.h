@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define NZ_ABI_VERSION 11
+#define NZ_ABI_VERSION 12
 
 enum nz_status {
     NZ_OK = 0,

@@ -41,6 +41,22 @@ def test_abi_version_matches_header_and_bindings():
     _native.lib()   # loads with the version check
 
 
+def test_a_library_from_before_the_escape_entries_is_refused_by_its_version(tmp_path, monkeypatch):
+    """Version 11's LUT images have other words in their escape entries and
+    its library no row products: the version check says so, before any
+    function that it lacks is looked up."""
+    source, stale = tmp_path / "stale.c", tmp_path / "libstale.so"
+    source.write_text("int nz_abi_version(void) { return 11; }\n")
+    try:
+        subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(stale)], check=True, capture_output=True)
+    except FileNotFoundError:
+        pytest.skip("no C compiler for the stale library")
+    monkeypatch.setattr(_native, "LIBRARY", stale)
+    monkeypatch.setattr(_native, "_lib", None)
+    with pytest.raises(ImportError, match="version 11"):
+        _native.lib()
+
+
 def test_descriptor_layouts_match_the_format_header(tmp_path):
     probe = tmp_path / "sizes.cpp"
     probe.write_text(
