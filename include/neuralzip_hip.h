@@ -134,7 +134,8 @@ int nz_layout_pack(const nz_layout* layout, uint8_t* dst, uint64_t dst_base,
  * others), segments 0 .. slots/2 - 1, whose workgroups are dispatched first
  * and win issue arbitration against the one sharing their unit, get
  * first_weight times the elements of the others. With segments == NULL only
- * *n_segments is set.
+ * *n_segments is set. Refuses coded tiles of more than 2048 elements, which a
+ * wavefront's staging area does not hold (of 32-bit words it holds 1024).
  * Replaces: the block->group / block->local id tensors (decoder.py:168-179). */
 int nz_plan_work(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_tiles, uint32_t slots,
                  double first_weight, nz_work* segments, uint32_t capacity, uint32_t* n_segments);

@@ -266,6 +266,17 @@ constexpr uint64_t kMinTilesPerGroup = 16;
 constexpr double kMaxRowExcess = 24576;
 constexpr size_t kXcds = 8;   // MI355X: accelerator dies, each with its own L2
 
+namespace {
+
+// A coded tile's `elements`, with `ahead` of them before it in its first
+// vector, must fit its wavefront's staging area.
+void check_staged(const nz_frag_desc& f, uint64_t ahead, uint32_t elements, uint32_t capacity) {
+    if (f.kind != NZ_KIND_RAW && ahead + elements > capacity)
+        fail(kLayoutLimit, "A coded tile exceeds the kernels' staging area.");
+}
+
+}  // namespace
+
 void check_matvec_group(const nz_matvec_weight* weights, uint32_t n_weights, uint32_t cols, unsigned element_size) {
     if (element_size != 2 && element_size != 4) fail(kInvalidArgument, "element_size must be 2 or 4.");
     if (!n_weights || n_weights > NZ_MATVEC_MAX_WEIGHTS) fail(kInvalidArgument, "A fused product takes 1 to 4 weights.");
@@ -305,6 +316,8 @@ void plan_matvec(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_til
         const nz_frag_desc& f = frags[tiles[t].frag];
         const uint64_t a0 = f.out + tiles[t].out0;
         const uint64_t a1 = a0 + nz_tile_elements(tiles[t].counts);
+        check_staged(f, a0 % (16 / element_size), nz_tile_elements(tiles[t].counts),
+                     nz_tile_capacity(static_cast<int>(element_size)));
         uint32_t w = 0;
         for (uint32_t k = 1; k < n_weights; ++k)
             if (a0 >= weights[k].offset) w = k;
@@ -356,6 +369,7 @@ void matvec_tiles(const nz_frag_desc* frags, uint32_t n_frags, const nz_tile* ti
         const uint64_t a0 = f.out + tile.out0;
         const uint64_t first = a0 / V * V, origin = f.out / V * V;
         const uint32_t elements = nz_tile_elements(tile.counts), windows = nz_tile_windows(tile.counts);
+        check_staged(f, a0 - first, elements, nz_tile_capacity(static_cast<int>(element_size)));
         // weight offsets are multiples of V, so `first` and a0 fall in the same weight (and row)
         uint32_t w = 0;
         for (uint32_t k = 1; k < n_weights; ++k)
@@ -451,7 +465,8 @@ Shares share_out(const nz_frag_desc* frags, const nz_tile* tiles, uint32_t n_til
             sum = 0;
         }
         if (t < n_tiles) {   // raw tiles only copy and merge: count them at half weight
-            const double n = nz_tile_elements(tiles[t].counts);
+            const uint32_t n = nz_tile_elements(tiles[t].counts);
+            check_staged(frags[tiles[t].frag], 0, n, NZ_TILE_OUT);   // (32-bit words: half; the plan does not know them)
             sum += frags[tiles[t].frag].kind == NZ_KIND_RAW ? 0.5 * n : n;
         }
     }

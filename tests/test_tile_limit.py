@@ -47,6 +47,44 @@ def test_tiles_hold_at_most_four_rounds(kind, dtype, offset):
         emulate_case(tensors, books, dtype)
 
 
+@pytest.mark.parametrize("dtype", sorted(LIMIT, key=str))
+@pytest.mark.parametrize("offset", [64, 67])
+def test_planners_refuse_coded_tiles_past_the_staging_area(dtype, offset):
+    """Tiles of a caller's own that a wavefront's staging area does not hold:
+    the record and row planners know the word's size and the tile's place in
+    its first vector, the launch planners only that no tile holds over 2048.
+    Raw tiles are not staged."""
+    es = DTYPES[dtype].element_size
+    limit, ahead = LIMIT[dtype], offset % (16 // es)
+    cols = 4096
+    descs, tiles = np.zeros(1, _native.FRAG_DESC), np.zeros(3, _native.TILE)
+    descs["kind"], descs["out"], descs["lane_stride"] = _native.KIND_SHORT, offset, 8192
+    weights = [(offset - ahead, 2)]
+
+    def plans(sizes):
+        tiles["n_out"], tiles["out0"] = sizes, np.concatenate([[0], np.cumsum(sizes)[:-1]])
+        _native.matvec_plan(descs, tiles, weights, cols, es)
+
+    def records(sizes):
+        tiles["n_out"], tiles["out0"] = sizes, np.concatenate([[0], np.cumsum(sizes)[:-1]])
+        _native.matvec_tiles(descs, tiles, weights, cols, es, 1 << 20)
+
+    for call in (plans, records):
+        with pytest.raises(_native.NativeError, match="staging area"):
+            call((limit - ahead + 1, 100, 100))
+        with pytest.raises(_native.NativeError, match="exactly once"):     # accepted so far
+            call((limit - ahead, 100, 100))
+    for call in (lambda: _native.plan_work(descs, tiles, 4), lambda: _native.plan_work_interleaved(descs, tiles, 4)):
+        descs["kind"] = _native.KIND_SHORT
+        tiles["n_out"] = (2049, 100, 100)
+        with pytest.raises(_native.NativeError, match="staging area"):
+            call()
+        descs["kind"] = _native.KIND_RAW
+        call()
+        descs["kind"], tiles["n_out"] = _native.KIND_SHORT, (2048, 100, 100)
+        call()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", sorted(LIMIT, key=str))
 @pytest.mark.parametrize("kind", ["limit", "windows"])
