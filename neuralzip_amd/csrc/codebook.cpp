@@ -373,6 +373,7 @@ unsigned lut_step(const std::vector<uint32_t>& lut, uint64_t window, uint32_t* b
         uint32_t shift = e & 31u, at = rest >> shift;
         if (at >= n) {
             const uint32_t second = (e >> NZ_ESC_SECOND) & 31u;
+            if (second >= shift) fail(kCorruptStream, "Escape entry does not lead to its code's token.");
             at = n + (rest >> second) - (n << (shift - second));
             shift = second;
         }

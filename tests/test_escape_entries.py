@@ -7,7 +7,7 @@ import torch
 
 import oracle
 from neuralzip_amd import _native
-from nz_helpers import segment_lengths, segment_tensor
+from nz_helpers import Encoded, segment_lengths, segment_tensor
 
 VOCAB = bytes((127, 127, 125, 126))
 PRIMARY, SEARCH = 4, 0     # first primary entry; word 0 of an entry that searches the records
@@ -87,6 +87,32 @@ def test_every_escape_entry_leads_to_its_code(name):
     if name == "spread-6-9-20":   # prefixes of one length, of two, and of more
         entries = [int(lut[PRIMARY + 2 * x]) for x in range(4096) if lut[PRIMARY + 2 * x] >> 27 == 0]
         assert {"search" if e == SEARCH else e >> 10 < 0xFFFF for e in entries} == {"search", True, False}
+
+
+@pytest.mark.parametrize("planted", ["lengths in falling order", "a shift of the whole word", "tokens moved"])
+def test_an_escape_entry_that_leads_elsewhere_raises(planted):
+    """A mistake planted in the entries of prefixes with two lengths must be
+    caught by the emulator's step, whatever the words say."""
+    book = BOOKS["spread-6-9-20"]
+    symbols = np.random.default_rng(4).permutation(np.repeat(np.arange(256), 20)).astype(np.uint8)
+    raw = segment_tensor(torch.bfloat16, symbols)
+    base, descs, tiles = Encoded([(raw, torch.bfloat16, 1 << 20, [0], 0)], {0: book}).host_image()
+    segments = _native.plan_work(descs, tiles, 4)
+    out = np.zeros(raw.size + 64, dtype=np.uint8)
+    _native.emulate_decode(base, descs, tiles, segments, 2, 1, out)
+    assert np.array_equal(out[:raw.size], raw)
+    image = base[int(descs["lut"][0]):].view(np.uint32)
+    two = [PRIMARY + 2 * x for x in range(4096) if image[PRIMARY + 2 * x] >> 27 == 0 and image[PRIMARY + 2 * x] != SEARCH
+           and image[PRIMARY + 2 * x] >> 10 < 0xFFFF]
+    assert two
+    for at in two:
+        first, second, n = int(image[at]) & 31, int(image[at]) >> 5 & 31, int(image[at]) >> 10
+        image[at] = {"lengths in falling order": second | first << 5 | n << 10,
+                     "a shift of the whole word": 0 | second << 5 | n << 10,
+                     "tokens moved": int(image[at])}[planted]
+        image[at + 1] += planted == "tokens moved"
+    with pytest.raises(_native.NativeError, match="Escape entry does not lead"):
+        _native.emulate_decode(base, descs, tiles, segments, 2, 1, out)
 
 
 @pytest.mark.gpu

@@ -13,7 +13,8 @@ import pytest
 
 HOST_TESTS = ["tests/test_corrupt_inputs.py", "tests/test_codec.py", "tests/test_reference_formats.py",
               "tests/test_abi.py", "tests/test_layout_emulator.py", "tests/test_setup_storage.py",
-              "tests/test_export_cpu.py", "tests/test_matvec.py", "tests/test_staging_scheme.py"]
+              "tests/test_export_cpu.py", "tests/test_matvec.py", "tests/test_staging_scheme.py",
+              "tests/test_row_products.py", "tests/test_escape_entries.py", "tests/test_tile_limit.py"]
 
 
 @pytest.fixture(scope="module")
