@@ -206,28 +206,27 @@ __device__ __forceinline__ Activations<BT> activations(const uint8_t* xp, uint32
 
 // The activations of rounds R0 to R1 - 1 of one tile, for this lane. Round r's
 // vector starts at column col0 + g of the tile's first row or, past its end,
-// of the next one: the smaller of the offset and the offset less a row, which
-// wraps round to a huge number in the first row. A tile of one row (most
-// tiles) needs one address for all rounds. Lanes past the tile read columns
-// that go unused.
+// of the next one. A tile of one row (most tiles) needs one address for all
+// rounds. Lanes past the tile read columns that go unused.
 template <int ES, int BT, uint32_t R0, uint32_t R1>
 __device__ __forceinline__ void fetch_x(const Activations<BT>& x, const RowSpan& rs, const TileInfo& ti, uint32_t cols,
                                         uint32_t lane, uint4 (*out)[BT]) {
+    constexpr uint32_t V = Geometry<ES>::V;
     const uint32_t at = rs.col0 * ES + lane * 16u;
     if (rs.split < ti.s1) {
         asm volatile("");
 #pragma unroll
         for (uint32_t r = R0; r < R1; ++r) {
-            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * Geometry<ES>::V) break;
+            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * V) break;
             const uint32_t a = at + r * NZ_WAVE * 16u;
 #pragma unroll
-            for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], min(a, a - cols * ES));
+            for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], nz_activation_offset(a - cols * ES, cols * ES));
         }
     } else {
         asm volatile("");
 #pragma unroll
         for (uint32_t r = R0; r < R1; ++r) {
-            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * Geometry<ES>::V) break;
+            if (late_round<ES>(r) && ti.s1 <= r * NZ_WAVE * V) break;
 #pragma unroll
             for (int b = 0; b < BT; ++b) out[r - R0][b] = load_vector(x.row[b], at + r * NZ_WAVE * 16u);
         }
@@ -238,7 +237,7 @@ template <int ES, int BT>
 __device__ __forceinline__ void fetch_x_round(const Activations<BT>& x, const RowSpan& rs, const TileInfo& ti,
                                               uint32_t cols, uint32_t lane, uint32_t r, uint4 (&out)[BT]) {
     const uint32_t a = rs.col0 * ES + lane * 16u + r * NZ_WAVE * 16u;
-    const uint32_t at = rs.split < ti.s1 ? min(a, a - cols * ES) : a;
+    const uint32_t at = rs.split < ti.s1 ? nz_activation_offset(a - cols * ES, cols * ES) : a;
 #pragma unroll
     for (int b = 0; b < BT; ++b) out[b] = load_vector(x.row[b], at);
 }

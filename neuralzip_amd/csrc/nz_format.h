@@ -148,6 +148,14 @@ struct nz_matvec_tile {          // 40 bytes
     uint32_t col0;               // column of the first vector's first element
 };
 
+// Byte offset in an activation row of `row_bytes` (under 2^32) of a vector
+// `past` bytes past the end of its tile's first row, mod 2^32: negative ones,
+// at most a tile's bytes before the end, lie in the first row, the others in
+// the next one.
+NZ_HD static inline uint32_t nz_activation_offset(uint32_t past, uint32_t row_bytes) {
+    return past + (row_bytes & static_cast<uint32_t>(static_cast<int32_t>(past) >> 31));
+}
+
 // A *row segment*: the work of one workgroup that owns output rows of a fused
 // product, so that it can add up its rows' partial sums itself. Its tiles
 // cover rows [row0, row1) of the stacked output; where a tile at either end
