@@ -10,6 +10,8 @@ output dtype. Repeated calls must give identical bits. Every partial sum
 the reduction reads must have been written: the partials buffer is poisoned
 with NaN first.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -530,19 +532,24 @@ def test_replace_switches_a_runtime_to_fused_products_and_back():
 
 
 @pytest.mark.gpu
-def test_matvec_on_a_side_stream_equals_the_current_stream():
+@pytest.mark.parametrize("form", ["rows", "two launches"])
+def test_matvec_on_a_side_stream_equals_the_current_stream(form):
     """HIPDecoder.matvec on a stream other than the current one, with its
     input a non-contiguous view (so the call makes its own copy), returns
     the bits of the same call on the current stream: while the current
     stream is still busy (the copy must be ordered on the launch stream) and
     while the launch stream is busy and the current stream allocates and
-    fills small blocks (the call's buffers must not be handed to it)."""
+    fills small blocks (the call's buffers must not be handed to it). In one
+    launch, and in two, whose partial sums the call allocates."""
     from neuralzip_amd.gpu.inference import NeuralZipRuntime, export_model_for_gpu
     from neuralzip_amd.setup import NeuralZipSetup
     model = BlockStack(depth=1).to(torch.bfloat16).eval()
     setup = NeuralZipSetup().build({n: p.detach() for n, p in model.named_parameters()})
     runtime = NeuralZipRuntime.attach(model, export_model_for_gpu(model, setup), device="cuda:0", matvec_tokens=1)
     plan = runtime._matvec["layers.0.up"]
+    assert plan.row_args[0] is not None
+    if form == "two launches":
+        plan = dataclasses.replace(plan, row_args=(None,) * len(plan.row_args))
     bias = model.layers[0].up.bias
     g = torch.Generator().manual_seed(6)
     wide = torch.randn(2048, 2, generator=g).to(torch.bfloat16).cuda()
@@ -562,6 +569,32 @@ def test_matvec_on_a_side_stream_equals_the_current_stream():
         current.wait_stream(side)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), busy
         del got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 2, 3, 4])
+def test_decoder_runs_the_form_that_fits_and_both_give_the_same_bits(batch):
+    """One workgroup for all rows, whose sums fit its LDS for one activation
+    row, not for two (16 staging areas), and again for three and four (12):
+    HIPDecoder.matvec takes the two launches where they do not fit, with its
+    own partial sums or the caller's, and either form gives the same bits."""
+    from neuralzip_amd.gpu.decoder import DeviceStore, default_decoder
+    rows, cols = 150, 4096
+    w = random_weight(torch.bfloat16, rows, cols, 12)
+    raw = w.view(torch.uint8).numpy().reshape(-1).copy()
+    book = _native.Codebook(singleton_header(raw, torch.bfloat16))
+    (layout, ids, *_), = Encoded([(raw, torch.bfloat16, raw.size // 2, [0], 0)], {0: book}).entries
+    store = DeviceStore({0: book}, [(layout, ids, 0)], torch.device("cuda:0"))
+    decoder, spec = default_decoder(), DTYPES[torch.bfloat16]
+    plan = decoder.prepare_matvec(store, [([0], 0, rows)], spec, cols, slots=1)
+    assert [a is not None for a in plan.row_args] == [True, False, True, True]
+    g = torch.Generator().manual_seed(batch)
+    x, bias = torch.randn(batch, cols, generator=g).to(torch.bfloat16), torch.randn(rows, generator=g).to(torch.bfloat16)
+    two = dataclasses.replace(plan, row_args=(None,) * len(plan.row_args))
+    partials = torch.full((2 * plan.n_tiles * batch,), float("nan"), device="cuda:0")
+    outs = [decoder.matvec(p, x.cuda(), [bias.cuda()], s)[0].cpu() for p in (plan, two) for s in (None, partials)]
+    check_product(outs[0], w, x, bias, torch.bfloat16)
+    assert all(torch.equal(o.view(torch.int16), outs[0].view(torch.int16)) for o in outs[1:])
 
 
 @pytest.mark.gpu
