@@ -443,8 +443,8 @@ __device__ __forceinline__ void decode_tile(LaneDecode l, const uint32_t* lut) {
 // (Reading the size first, then copying in a loop that waits for each of its
 // loads, put four memory latencies one after the other ahead of a
 // workgroup's first tile; two are left. With the decode kernel's first tiles
-// requested beside it, 14.9 M bf16 elements went from 11.9 to 10.3 us and
-// 13.1 M fp32 elements from 18.2 to 17.5.)
+// requested beside it, 14.9 M bf16 elements went from 11.0 to 10.7 us of
+// kernel time and 13.1 M fp32 elements from 17.8 to 16.9.)
 template <bool REORDER, int THREADS>
 struct LutCopy {
     static constexpr uint32_t kPrimary = NZ_LUT_ENTRIES / 2;   // 16-byte vectors of two entries

@@ -39,8 +39,8 @@
 // lanes x 8 elements. 64 windows of N(0, std^2) bf16 weights hold about 1600
 // elements, of uniform ones 2048. A limit of 1536 (three rounds) spares the
 // former the fourth round's few lanes (28672 x 4096 bf16 product 41.6 us
-// against 43.8), but takes lanes from codes under two bits: the same product
-// with 90 % zeros 57.2 against 47.8, ternary 46.2 against 39.5; 14.9 M ternary
+// against 43.0), but takes lanes from codes under two bits: the same product
+// with 90 % zeros 57.2 against 48.0, ternary 46.2 against 39.5; 14.9 M ternary
 // weights decoded 10.6 against 9.1, 277 M equal ones 287 against 274.
 #define NZ_TILE_OUT 2048
 #define NZ_TILE_OUT32 1024        // the same for 32-bit words

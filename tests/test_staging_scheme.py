@@ -1,4 +1,4 @@
-"""The staging stores of the gfx950 tile decode (stage_tile in
+"""The staging stores of the gfx950 tile decode (decode_tile in
 neuralzip_amd/csrc/hip/tile_decode.h), simulated on the CPU in lockstep.
 
 The wavefront clears its staging area; then each lane decodes its window's
